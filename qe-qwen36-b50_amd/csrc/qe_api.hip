@@ -157,7 +157,7 @@ int qe_moe_create(int device, int n_layers, int t_max, qe_moe_ctx **out) {
     A(S.xhl, T32 * QE_D * 4);
     A(S.logits, T * QE_ROUTER_ROWS * 4);
     A(S.shgu, T32 * QE_FF_SH * 4);
-    A(S.rpart, 8 * T * QE_N_EXPERT * 4);
+    A(S.rpart, qe_rpart_rows(T) * QE_N_EXPERT * 4);
     A(S.ids, NP * 4);
     A(S.wts, NP * 4);
     A(S.shg, T * 4);

@@ -6,7 +6,23 @@
 #include "qe_device.h"
 
 #define QE_SMALL_T 8   /* calls of up to this many tokens take the persistent decode kernel */
-#define RT_SPLIT 8     /* router K split: subtrees of 64 / RT_SPLIT chunks, merged by k_topk */
+// The router's K splits at T tokens (subtrees of 64 / nz chunks, whose partials
+// k_topk merges): enough workgroups of 64 tokens x 128 experts to fill the GPU, and
+// no more, since every split writes T x 256 partials (8192 tokens: 4 splits 96 + 13 us
+// with k_topk, 8 splits 102 + 18; 1999: 8 splits 32 + 7, 16 splits 39 + 9; 512 in the
+// fused launch: 16 splits 21.3, 32 splits 25).
+// From QE_RS_SPLIT_T tokens the router and the shared gate/up tiles run as two
+// launches of larger tiles (1024 tokens: 43 us fused, 47 apart; 1999: 88 against 67).
+#define QE_RS_SPLIT_T 1280
+static inline int qe_router_splits(int T) { return T < 256 ? 32 : T < QE_RS_SPLIT_T ? 16 : T < 4096 ? 8 : 4; }
+static inline size_t qe_rpart_rows(size_t t_max) { // token rows of partials that calls of up to t_max tokens write
+    size_t n = 0;
+    for (size_t end : {(size_t)255, (size_t)QE_RS_SPLIT_T - 1, (size_t)4095, t_max}) {
+        const size_t t = end < t_max ? end : t_max, rows = t * qe_router_splits((int)t);
+        n = n > rows ? n : rows;
+    }
+    return n;
+}
 #define QE_MFMA_MC 64 /* pairs per work item of the prefill MFMA grouped GEMMs (up to four 16-row tiles) */
 
 
@@ -54,7 +70,7 @@ struct QeScratch {
     _Float16 *xhl;                          // [T][2048] normed x as fp16 hi|lo halves (store_hilo16 layout)
     float *logits;                          // [T][257]
     float *shgu;                            // prefill: shared silu(g)*u as [T][512] fp16 hi|lo halves
-    float *rpart;                           // [8][T][256] router subtree partials
+    float *rpart;                           // [nz][T][256] router subtree partials (qe_router_splits)
     int32_t *ids; float *wts; float *shg;   // [T][8], [T][8], [T]
     int32_t *off; int32_t *pairs;           // [257], [T*8]
     int4 *items; int32_t *n_items;          // work items (expert, first pair, count); n_items[0] items, the first n_items[1] big

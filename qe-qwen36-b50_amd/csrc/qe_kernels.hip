@@ -118,15 +118,14 @@ __global__ __launch_bounds__(64 * NQ_TOK) void k_normq(const float *x, int T, co
     lane_quant_store_opnd(v, xqp + (size_t)t * QE_D, lane, xs + (size_t)t * (QE_D / 32) + lane);
 }
 
-static_assert(RT_SPLIT == 8, "k_topk merges eight router partials");
-
-// Wave per token, 4 tokens per workgroup: logits (router partials merged +
-// bias; row 256 came from k_normq), then top-8 (the survivors of a group-maximum
+// Wave per token, 4 tokens per workgroup: logits (the router's NZ subtree partials
+// merged, the tree's top levels, + bias; row 256 came from k_normq), then top-8 (the survivors of a group-maximum
 // threshold sorted in registers), weights and the shared gate
 // (engine/qe.cpp:1454-1483).  The workgroup then adds its 32 expert ids
 // to the dispatch histogram of its 1024-pair chunk (zeroed by k_normq), one
 // global add per distinct expert.
-__global__ __launch_bounds__(256) void k_topk(const float *part, const float *bias, int T, float *logits, int32_t *ids,
+template <int NZ>
+__global__ __launch_bounds__(256) void k_topk(const float *part, const float *bias, float *logits, int T, int32_t *ids,
                                               float *wts, float *shg, int32_t *chunk_hist) {
     __shared__ int s_h[QE_N_EXPERT];
     __shared__ uint64_t s_sk[4][64]; // each wave's survivor keys
@@ -134,21 +133,24 @@ __global__ __launch_bounds__(256) void k_topk(const float *part, const float *bi
     if (threadIdx.x < QE_N_EXPERT) s_h[threadIdx.x] = 0;
     __syncthreads();
     if (t < T) {
-    const size_t n = (size_t)T * QE_N_EXPERT;
+    float *lr = logits + (size_t)t * QE_ROUTER_ROWS;
     float v[4];
+    float p[4][NZ];
+#pragma unroll
+    for (int z = 0; z < NZ; ++z)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) p[j][z] = part[((size_t)z * T + t) * QE_N_EXPERT + lane + 64 * j];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int e = lane + 64 * j;
-        const float *p = part + (size_t)t * QE_N_EXPERT + e;
-        float s[8];
 #pragma unroll
-        for (int z = 0; z < 8; ++z) s[z] = p[z * n];
-        float x = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
-        if (bias) x = x + bias[e];
-        v[j] = x;
-        logits[(size_t)t * QE_ROUTER_ROWS + e] = x;
+        for (int n = NZ / 2; n >= 1; n /= 2)
+#pragma unroll
+            for (int z = 0; z < n; ++z) p[j][z] = p[j][2 * z] + p[j][2 * z + 1];
+        v[j] = p[j][0];
+        if (bias) v[j] = v[j] + bias[lane + 64 * j];
+        lr[lane + 64 * j] = v[j];
     }
-    const float lg = logits[(size_t)t * QE_ROUTER_ROWS + QE_N_EXPERT];
+    const float lg = lr[QE_N_EXPERT];
     const int e = wave_topk_sorted(v, lg, lane, s_sk[threadIdx.x >> 6], ids + t * QE_K_USED, wts + t * QE_K_USED, shg + t);
     if (lane < QE_K_USED) atomicAdd(&s_h[e], 1);
     }
@@ -410,7 +412,15 @@ hipError_t qe_launch_layer(const QeLayerPtrs &L, const QeScratch &S, const float
     }
     {
         QE_PROF(QP_TOPK);
-        k_topk<<<(T + 3) / 4, 256, 0, st>>>(S.rpart, L.bias, T, S.logits, S.ids, S.wts, S.shg, S.chunk_hist);
+        const auto go = [&](auto kern) {
+            kern<<<(T + 3) / 4, 256, 0, st>>>(S.rpart, L.bias, S.logits, T, S.ids, S.wts, S.shg, S.chunk_hist);
+        };
+        switch (qe_router_splits(T)) {
+        case 4: go(k_topk<4>); break;
+        case 8: go(k_topk<8>); break;
+        case 16: go(k_topk<16>); break;
+        default: go(k_topk<32>); break;
+        }
     }
     {
         QE_PROF(QP_DISPATCH); // the histogram came with k_topk

@@ -613,16 +613,16 @@ __global__ __launch_bounds__(256, 4) void k_expert_gu(GemmTileArgs a) {
 // The activations are stored in exactly that order (qe_hl_off), so each of a
 // lane's four A chunks per block is one 1 KB-contiguous dwordx4 load, and its
 // B operand is one 16-byte run of a Q8 row.
-//   gate/up: workgroup = 32 tokens x (gate rows j0..j0+31, up rows j0..j0+31),
-//            the four waves split K in quarters, partial sums meet in LDS,
-//            h = silu(g) * u is written as hi|lo halves (below 2048 tokens;
-//            from there shgu_tile64).
+//   gate/up: workgroup = 32 tokens x (gate rows j0..j0+15, up rows j0..j0+15),
+//            the eight waves split K in eighths, partial sums meet in LDS,
+//            h = silu(g) * u is written as hi|lo halves (below QE_RS_SPLIT_T
+//            tokens; from there shgu_tile64).
 //   down:    workgroup = 64 tokens x 128 output rows, LDS-staged (shdn_tile64).
 // Rows T..T+31 of the last tile exist in the buffers (sized for whole tiles) and
 // are never stored; each output row depends on its own A row only.
 // ===========================================================================
 typedef float qe_float16v __attribute__((ext_vector_type(16)));
-#define SH_GU_KB 16 /* 32-blocks per wave in gate/up: 2048 / 32 / 4 */
+#define SH_GU_KB 8 /* 32-blocks per wave in gate/up: 2048 / 32 / 8 */
 
 QE_DEV qe_u32x4 sh_ld(__amdgpu_buffer_rsrc_t r, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0); }
 
@@ -642,140 +642,173 @@ QE_DEV void sh_block(const qe_u32x4 a[4], qe_u32x4 w, float dw, qe_float16v &acc
     // keeping all the block products live
     asm volatile("" : "+v"(acc));
 }
-QE_DEV float half_of(const qe_u32x4 s[2], int b) { // fp16 scale b of 16 packed in two dwordx4
-    const uint32_t w = s[b >> 3][(b >> 1) & 3];
+QE_DEV float half_of(qe_u32x4 s, int b) { // fp16 scale b of 8 packed in a dwordx4
+    const uint32_t w = s[b >> 1];
     return f16_bits_to_f32((uint16_t)((b & 1) ? w >> 16 : w & 0xffffu));
 }
 
-// Router logits 0..255 in the canonical fp32 order, tiled:
-// C[m][n] = sum_k xn[m][k] W[n][k].  Canonical order: per 32-wide k chunk an fma
-// chain from 0, chunk sums merged by the pairwise tree (chunks (c, c+1), then
-// pairs of pairs, ...).  The K range is split eight ways along that tree: split
-// z computes the 8-chunk subtree [8z, 8z+8) exactly, and k_topk forms the top
-// three levels ((s0 + s1) + (s2 + s3)) + ((s4 + s5) + (s6 + s7)) -- bit-identical
-// to the unsplit order.  Row 256 (the shared-expert gate) is one canonical wave
-// dot per token in k_normq.  Tile 64 tokens x 64 rows, 256 threads, 4 x 4 outputs
-// per thread; chunks are double-buffered in LDS, k-major, the next one loaded
-// into registers while the current one is multiplied.  The transposing stores
-// XOR the column with the k group ((k / 8) % 4 * 16), so the four k groups a
-// wave stores land in different banks; the reads undo it (float4 runs stay
-// aligned).
-struct RouterSmem {
-    float As[2][32][64];
-    float Bs[2][32][64];
+// Router logits 0..255 on the fp32 matrix cores, in the canonical order: per
+// 32-wide k chunk an fma chain from 0 in ascending k, chunk sums merged by the
+// pairwise tree (chunks (c, c+1), then pairs of pairs, ...).  The chain is what
+// v_mfma_f32_32x32x2_f32 computes: each output is accumulated k by k with one
+// rounding per step, bit-identical to the fmaf chain (checked on the GPU over
+// normal, subnormal, overflowing and special values), at 32 fp32 multiply-adds per
+// cycle and SIMD where v_fma_f32 reaches 16.  The K range is split along the tree:
+// split z computes the subtree of chunks [z 2^LEV, (z + 1) 2^LEV), keeping the
+// levels' sums in registers by a binary counter, and k_topk forms the top levels
+// and adds the bias -- bit-identical to the unsplit order.  Row 256 (the
+// shared-expert gate) is one canonical wave dot per token in k_normq.
+//
+// LDS of router_tile: two stages of one 32-wide k chunk of the tile's rows (64
+// tokens, then the experts), 128 bytes a row.  Within eight k the even ones come
+// first (run 2 o: k 8 o + 0, 2, 4, 6), then the odd ones (run 2 o + 1), so one
+// 16-byte read gives a lane (half h) its operands of four steps, k = 2 s + h, with
+// no lane swaps (VALU work beside the matrix instructions hides only by half).  Run
+// q of row r sits at run q ^ (r / 2 % 8): the 16 rows a lane group reads in one
+// instruction fall in sixteen different bank groups.
+template <int NE> struct RouterSmem {
+    alignas(16) uint8_t st[2][64 + 32 * NE][128];
 };
-QE_DEV void router_tile(const float *xn, int T, const float *W, float *part, int n_tile, int m_tile, int z,
-                        RouterSmem &sm) {
-    constexpr int NCH = 64 / RT_SPLIT; // chunks per split
-    auto &As = sm.As;
-    auto &Bs = sm.Bs;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int m0 = m_tile * 64, n0 = n_tile * 64;
-    const int lr = tid >> 2, lk = (tid & 3) * 8; // loader: row lr of the tile, 8 k values
-    const bool a_ok = m0 + lr < T;
-    const float *ap = xn + (size_t)(a_ok ? m0 + lr : 0) * QE_D + z * NCH * 32 + lk;
-    const float *bp = W + (size_t)(n0 + lr) * QE_D + z * NCH * 32 + lk;
-    float4 pa[2], pb[2];
-    auto fetch = [&](int cl) {
-        const float4 *a4 = (const float4 *)(ap + cl * 32), *b4 = (const float4 *)(bp + cl * 32);
-        pa[0] = a_ok ? a4[0] : make_float4(0.f, 0.f, 0.f, 0.f);
-        pa[1] = a_ok ? a4[1] : make_float4(0.f, 0.f, 0.f, 0.f);
-        pb[0] = b4[0];
-        pb[1] = b4[1];
-    };
-    auto stage = [&](int buf) {
-        const float va[8] = {pa[0].x, pa[0].y, pa[0].z, pa[0].w, pa[1].x, pa[1].y, pa[1].z, pa[1].w};
-        const float vb[8] = {pb[0].x, pb[0].y, pb[0].z, pb[0].w, pb[1].x, pb[1].y, pb[1].z, pb[1].w};
-        const int col = lr ^ ((lk >> 3) << 4);
+// Tile 64 tokens x 32 NE experts: wave w takes tokens 32 (w % 2) + 0..31 and NT
+// 32-expert tiles from 32 NT (w / 2); NT = 2 feeds two matrix instructions with
+// every token operand, NT = 1 makes twice the waves.
+template <int LEV, int NE, int NT>
+QE_DEV void router_tile(const float *xn, int T, const float *W, float *part, int m_tile, int n_tile, int z,
+                        RouterSmem<NE> &sm) {
+    constexpr int NCH = 1 << LEV, NWV = 2 * NE / NT, NR = (8 + 4 * NE) / NWV; // NR: staging instructions per wave
+    static_assert(LEV >= 1 && NR * NWV == 8 + 4 * NE, "chunks in pairs; eight rows per staging instruction");
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 31, h = lane >> 5;
+    const int m0 = m_tile * 64, n0 = n_tile * 32 * NE;
+    // staging: wave w brings rows 8 NR w .. 8 NR (w + 1) - 1, eight rows (whole
+    // 128-byte lines) per instruction, a chunk ahead in registers.  (Loads straight
+    // into LDS would be drained before the next LDS read of either stage.)
+    // Range-checked buffers from the tile's first token row and expert row: a row
+    // past T reads zeros and is never stored.
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(xn + (size_t)m0 * QE_D), (short)0, (T - m0) * QE_D * 4, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rw =
+        __builtin_amdgcn_make_buffer_rsrc((void *)(W + (size_t)n0 * QE_D), (short)0, 32 * NE * QE_D * 4, 0x00020000);
+    const uint32_t vo = (lane >> 3) * (QE_D * 4) + 16 * (lane & 7);
+    // of the lane's four k (half u of eight k o): 0 and 2 go to run 2 o, 1 and 3 to run
+    // 2 o + 1 (the next run up or down after the swizzle), from float 2 u of the run
+    const uint32_t dst = 128 * (lane >> 3) + 16 * ((lane & 6) ^ (lane >> 4)) + 8 * (lane & 1);
+    qe_u32x4 stg[NR];
+    auto fetch = [&](int c) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            As[buf][lk + i][col] = va[i];
-            Bs[buf][lk + i][col] = vb[i];
+        for (int j = 0; j < NR; ++j) {
+            const int i = NR * wv + j; // rows 8 i .. 8 i + 7 of the tile: tokens, then experts
+            stg[j] = __builtin_amdgcn_raw_buffer_load_b128(i < 8 ? rx : rw, vo + (i & 7) * (8 * QE_D * 4) + (i >= 16) * (64 * QE_D * 4),
+                                                           (z * NCH + c) * 128, 0);
         }
+    };
+    auto put = [&](int s) {
+#pragma unroll
+        for (int j = 0; j < NR; ++j) {
+            const int i = NR * wv + j;
+            uint8_t *row = &sm.st[s][0][0] + 1024 * i;
+            uint32_t *ev = (uint32_t *)(row + (dst ^ (64 * (i & 1)))), *od = (uint32_t *)(row + (dst ^ (64 * (i & 1)) ^ 16));
+            ev[0] = stg[j].x;
+            ev[1] = stg[j].z;
+            od[0] = stg[j].y;
+            od[1] = stg[j].w;
+        }
+    };
+    const int ra = 32 * (wv & 1) + r, rb = 64 + 32 * NT * (wv >> 1) + r; // this lane's rows: tokens, experts (and rb + 32)
+    const int sw = (r >> 1) & 7;                                         // (all swizzle alike)
+    qe_u32x4 raw[2][1 + NT];                                             // operands of four steps, by parity of the run pair
+    auto read = [&](int stage, int q) {
+        const int off = 16 * ((2 * q + h) ^ sw);
+#pragma unroll
+        for (int o = 0; o < 1 + NT; ++o)
+            raw[q & 1][o] = *(const qe_u32x4 *)(&sm.st[stage][0][0] + 128 * (o == 0 ? ra : rb + 32 * (o - 1)) + off);
     };
     fetch(0);
-    stage(0);
+    put(0);
+    fetch(1);
     __syncthreads();
-    float st[4][4][4];
-#pragma unroll 1
-    for (int cl = 0; cl < NCH; ++cl) {
-        const int buf = cl & 1;
-        if (cl + 1 < NCH) fetch(cl + 1);
-        float acc[4][4];
+    read(0, 0);
+    // One chunk: the operands of run pair q + 1 are read from LDS before the matrix
+    // instructions of q are issued.  The next chunk is put into the other stage after
+    // pair 2 (that stage's last reads were issued before the previous barrier), and
+    // its first operands are read behind the barrier, ahead of pair 3.
+    auto chunk = [&](int c, int stage, qe_float16v (&acc)[NT]) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int t = 0; t < NT; ++t) acc[t] = qe_float16v{};
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+        for (int q = 0; q < 4; ++q) {
+            if (q == 3) {
+                put(stage ^ 1); // past the last chunk: nothing reads it
+                __syncthreads();
+                fetch(c + 2 < NCH ? c + 2 : NCH - 1);
+            }
+            read(q == 3 ? stage ^ 1 : stage, (q + 1) & 3);
+            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int kk = 0; kk < 32; ++kk) {
-            const int sw = ((kk >> 3) & 3) << 4;
-            const float4 av = *(const float4 *)&As[buf][kk][(ty * 4) ^ sw];
-            const float4 bv = *(const float4 *)&Bs[buf][kk][(tx * 4) ^ sw];
-            const float ar[4] = {av.x, av.y, av.z, av.w}, br[4] = {bv.x, bv.y, bv.z, bv.w};
+            for (int s = 0; s < 4; ++s)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(ar[i], br[j], acc[i][j]);
+                for (int t = 0; t < NT; ++t)
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(raw[q & 1][0][s]),
+                                                                  __uint_as_float(raw[q & 1][1 + t][s]), acc[t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        bool carry = true; // pairwise-tree merge of chunk cl
+    };
+    qe_float16v a0[NT], acc[NT], st[LEV][NT]; // st[l]: level l sum waiting for its sibling (level 0 is a0)
+#pragma unroll 1
+    for (int c = 0; c < NCH; c += 2) {
+        chunk(c, 0, a0);
+        chunk(c + 1, 1, acc);
 #pragma unroll
-        for (int l = 0; l < 4; ++l) {
+        for (int t = 0; t < NT; ++t) acc[t] = a0[t] + acc[t];
+        bool carry = true; // pairwise-tree merge of the chunk pair
+#pragma unroll
+        for (int l = 1; l < LEV; ++l) {
             if (carry) {
-                if (cl & (1 << l)) {
+                if (c & (1 << l)) {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) acc[i][j] = st[l][i][j] + acc[i][j];
+                    for (int t = 0; t < NT; ++t) acc[t] = st[l][t] + acc[t];
                 } else {
 #pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) st[l][i][j] = acc[i][j];
+                    for (int t = 0; t < NT; ++t) st[l][t] = acc[t];
                     carry = false;
                 }
             }
         }
-        if (cl + 1 < NCH) stage(buf ^ 1);
-        __syncthreads();
     }
-    constexpr int TOP = NCH == 8 ? 3 : NCH == 16 ? 4 : 2;
+    // the last pair's merge carried through every level: acc is the subtree's sum
+    float *out = part + ((size_t)z * T + m0) * QE_N_EXPERT + n0 + 32 * NT * (wv >> 1) + r;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= T) continue;
-        *(float4 *)&part[((size_t)z * T + m) * QE_N_EXPERT + n0 + tx * 4] =
-            make_float4(st[TOP][i][0], st[TOP][i][1], st[TOP][i][2], st[TOP][i][3]);
-    }
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int m = 32 * (wv & 1) + 8 * (i >> 2) + 4 * h + (i & 3);
+            if (m0 + m < T) out[m * QE_N_EXPERT + 32 * t] = acc[t][i];
+        }
 }
 
 struct ShguSmem {
-    float red[4][2][16][64];
+    float red[8][16][64]; // [K eighth][accumulator register][lane]
 };
+// 32 tokens x 16 h columns: the 32 columns of the matrix tile are the 16 gate rows
+// j0.. and the 16 up rows, wave w takes blocks 8 w .. 8 w + 7 of K.
 QE_DEV void shgu_tile(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *hhl, int m_tile, int j_tile, ShguSmem &sm) {
     constexpr uint32_t RB = QE_SH_GU_ROW_BYTES;
     auto &red = sm.red;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c = lane & 31, kh = lane >> 5;
-    const int m0 = m_tile * 32, j0 = j_tile * 32, kb0 = wv * SH_GU_KB;
+    const int m0 = m_tile * 32, j0 = j_tile * 16, kb0 = wv * SH_GU_KB;
     const __amdgpu_buffer_rsrc_t ra =
         __builtin_amdgcn_make_buffer_rsrc((void *)xhl, (short)0, ((T + 31) & ~31) * QE_D * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)W, (short)0, (int)QE_SH_GU_BYTES, 0x00020000);
     const uint32_t a_off = (uint32_t)(m_tile * (QE_D / 32) + kb0) * 4096 + lane * 16;
-    const uint32_t g_off = (uint32_t)(j0 + c) * RB, u_off = g_off + QE_FF_SH * RB;
-    qe_u32x4 sg[2], su[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        sg[i] = sh_ld(rw, g_off + QE_D + 2 * kb0 + 16 * i);
-        su[i] = sh_ld(rw, u_off + QE_D + 2 * kb0 + 16 * i);
-    }
-    qe_float16v ag = {}, au = {};
+    const uint32_t w_off = (uint32_t)((c >> 4) * QE_FF_SH + j0 + (c & 15)) * RB;
+    const qe_u32x4 sc = sh_ld(rw, w_off + QE_D + 2 * kb0); // the eight blocks' scales
+    qe_float16v acc = {};
     constexpr int DEPTH = 3;
-    qe_u32x4 ra_[DEPTH][4], rg[DEPTH], ru[DEPTH];
+    qe_u32x4 ra_[DEPTH][4], rb[DEPTH];
     auto load = [&](int b) {
         const int s = b % DEPTH;
 #pragma unroll
         for (int q = 0; q < 4; ++q) ra_[s][q] = sh_ld(ra, a_off + 4096 * b + 1024 * q);
-        rg[s] = sh_ld(rw, g_off + 32 * (kb0 + b) + 16 * kh);
-        ru[s] = sh_ld(rw, u_off + 32 * (kb0 + b) + 16 * kh);
+        rb[s] = sh_ld(rw, w_off + 32 * (kb0 + b) + 16 * kh);
     };
 #pragma unroll
     for (int b = 0; b < DEPTH; ++b) load(b);
@@ -783,55 +816,53 @@ QE_DEV void shgu_tile(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *hh
     for (int b = 0; b < SH_GU_KB; ++b) {
         const int s = b % DEPTH;
         const qe_u32x4 a[4] = {ra_[s][0], ra_[s][1], ra_[s][2], ra_[s][3]};
-        const qe_u32x4 wg = rg[s], wu = ru[s];
+        const qe_u32x4 w = rb[s];
         if (b + DEPTH < SH_GU_KB) load(b + DEPTH);
-        sh_block(a, wg, half_of(sg, b), ag);
-        sh_block(a, wu, half_of(su, b), au);
+        sh_block(a, w, half_of(sc, b), acc);
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        red[wv][0][i][lane] = ag[i];
-        red[wv][1][i][lane] = au[i];
-    }
+    for (int i = 0; i < 16; ++i) red[wv][i][lane] = acc[i];
     __syncthreads();
-    // thread: lane L of the accumulators, i = 4 (tid / 64) .. +3 -> 4 (token, j) outputs
+    {   // thread: register i = 2 (tid / 64) + half of the wave, token row kh2, column j
+        const int i = 2 * wv + (lane >> 5), k2 = (lane >> 4) & 1, j = lane & 15;
+        float p[2][8];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        const int i = 4 * wv + q;
-        const float g = (red[0][0][i][lane] + red[1][0][i][lane]) + (red[2][0][i][lane] + red[3][0][i][lane]);
-        const float u = (red[0][1][i][lane] + red[1][1][i][lane]) + (red[2][1][i][lane] + red[3][1][i][lane]);
-        const int m = m0 + 8 * (i >> 2) + 4 * kh + (i & 3), j = j0 + c;
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int w = 0; w < 8; ++w) p[u][w] = red[w][i][32 * k2 + 16 * u + j];
+        const float g = ((p[0][0] + p[0][1]) + (p[0][2] + p[0][3])) + ((p[0][4] + p[0][5]) + (p[0][6] + p[0][7]));
+        const float u = ((p[1][0] + p[1][1]) + (p[1][2] + p[1][3])) + ((p[1][4] + p[1][5]) + (p[1][6] + p[1][7]));
+        const int m = m0 + 8 * (i >> 2) + 4 * k2 + (i & 3);
         if (m < T) {
             const float h = silu_mul(g, u);
             const _Float16 hi = (_Float16)h, lo = (_Float16)(h - (float)hi);
-            uint8_t *dst = (uint8_t *)hhl + qe_hl_off(QE_FF_SH, m, j);
+            uint8_t *dst = (uint8_t *)hhl + qe_hl_off(QE_FF_SH, m, j0 + j);
             *(_Float16 *)dst = hi;
             *(_Float16 *)(dst + QE_HL_LO) = lo;
         }
     }
 }
 
-
-// Router split tiles and shared gate/up tiles in one launch, so the fp32 VALU
-// router and the matrix-core shared GEMM share the CUs instead of running back
-// to back.  Workgroup b runs on XCD b % 8 (the dispatcher deals workgroups
+// Router tiles and shared gate/up tiles in one launch of 512-thread workgroups:
+// neither fills the GPU alone below QE_RS_SPLIT_T tokens, and each launch costs
+// about 4.5 us.  Workgroup b runs on XCD b % 8 (the dispatcher deals workgroups
 // round robin over the 8 XCDs, each with its own L2), and the tasks are dealt
 // so that every XCD gets both kinds, interleaved, and the tiles that share an
-// operand run on one XCD back to back: the 4 router column tiles of one
-// (token tile, K split) and the 16 shared gate/up row tiles of one token tile.
-constexpr int RS_NT = QE_N_EXPERT / 64, RS_JT = QE_FF_SH / 32;
-QE_DEV int rs_router_per_xcd(int T) { return RS_NT * ((T + 63) / 64) * RT_SPLIT / 8; }
-QE_DEV int rs_shgu_per_xcd(int T, int x) { return RS_JT * (((T + 31) / 32 - x + 7) / 8); }
-__global__ __launch_bounds__(256) void k_router_shgu(const float *xn, const _Float16 *xhl, int T, const float *Wr,
-                                                     const uint8_t *Wg, float *part, _Float16 *hhl) {
+// operand run on one XCD back to back: the two router column tiles of one (token
+// tile, K split) and the 32 shared gate/up row tiles of one token tile.
+constexpr int RS_JT = QE_FF_SH / 16;
+QE_HD int rs_router_per_xcd(int T, int nz, int x) { return 2 * (((T + 63) / 64 * nz - x + 7) / 8); }
+QE_HD int rs_shgu_per_xcd(int T, int x) { return RS_JT * (((T + 31) / 32 - x + 7) / 8); }
+template <int LEV>
+__global__ __launch_bounds__(512, 4) void k_router_shgu(const float *xn, const _Float16 *xhl, int T, const float *Wr,
+                                                        const uint8_t *Wg, float *part, _Float16 *hhl) {
     __shared__ union {
-        RouterSmem r;
+        RouterSmem<4> r;
         ShguSmem s;
     } sm;
-    static_assert(RT_SPLIT % 8 == 0, "router groups divide evenly over the XCDs");
+    constexpr int NZ = 64 >> LEV;
     const int x = blockIdx.x & 7, k = blockIdx.x >> 3;
-    const int mt64 = (T + 63) / 64;
-    const int nr = rs_router_per_xcd(T), ns = rs_shgu_per_xcd(T, x), both = 2 * (nr < ns ? nr : ns);
+    const int nr = rs_router_per_xcd(T, NZ, x), ns = rs_shgu_per_xcd(T, x), both = 2 * (nr < ns ? nr : ns);
     bool router;
     int idx;
     if (k < both) {
@@ -843,61 +874,60 @@ __global__ __launch_bounds__(256) void k_router_shgu(const float *xn, const _Flo
     }
     if (router) {
         if (idx >= nr) return;
-        const int g = 8 * (idx / RS_NT) + x; // (token tile, K split) group
-        router_tile(xn, T, Wr, part, idx % RS_NT, g % mt64, g / mt64, sm.r);
+        const int g = 8 * (idx >> 1) + x;
+        router_tile<LEV, 4, 1>(xn, T, Wr, part, g / NZ, idx & 1, g % NZ, sm.r);
     } else {
         if (idx >= ns) return;
         shgu_tile(xhl, T, Wg, hhl, 8 * (idx / RS_JT) + x, idx % RS_JT, sm.s);
     }
 }
 
-// From QE_RS_SPLIT_T tokens on, the two kinds run as two launches instead: the
-// shared gate/up tiles hold 128 AGPRs, which caps the fused kernel at 2 waves
-// per SIMD, while the router tiles alone (128 VGPRs) run 4.  One wave issues a
-// VALU instruction only every ~5 cycles, so the fp32 router needs the waves
-// (8192 tokens: fused 266 us; router 117 + shared 131 us).  At 512 tokens the
-// fused launch is 9 us faster (20 against 17 + 12).
-#define QE_RS_SPLIT_T 2048
-__global__ __launch_bounds__(256) void k_router(const float *xn, int T, const float *Wr, float *part) {
-    __shared__ RouterSmem sm;
-    const int x = blockIdx.x & 7, k = blockIdx.x >> 3, mt64 = (T + 63) / 64;
-    const int g = 8 * (k / RS_NT) + x;
-    router_tile(xn, T, Wr, part, k % RS_NT, g % mt64, g / mt64, sm);
+// From QE_RS_SPLIT_T tokens on, two launches with larger tiles.
+// workgroup b on XCD b % 8: the two expert tiles of a (token tile, K split) back to back there
+template <int LEV> __global__ __launch_bounds__(256, 2) void k_router(const float *xn, int T, const float *Wr, float *part) {
+    __shared__ RouterSmem<4> sm;
+    constexpr int NZ = 64 >> LEV;
+    const int x = blockIdx.x & 7, k = blockIdx.x >> 3, g = 8 * (k >> 1) + x;
+    if (g >= (T + 63) / 64 * NZ) return;
+    router_tile<LEV, 4, 2>(xn, T, Wr, part, g / NZ, k & 1, g % NZ, sm);
 }
 // Shared gate/up for large T: workgroup = 64 tokens (two 32-token tiles) x 64
-// gate rows + the same 64 up rows; wave w takes token tile w & 1 and rows
-// 32 (w >> 1) + 0..31 of both, over the full K, so no partial sums meet.  Each
-// 32-block of K, the workgroup stages the 8 KB of activations and 4 KB of Q8
-// rows in LDS once (double-buffered, one barrier per block) and every wave reads
-// its operands from there: each fetched byte feeds two waves' MFMAs instead of
-// one.  The Q8 block scales of the 128 rows sit in LDS for the whole K, block-
-// major, so the 32 rows a wave reads for one block are consecutive.
-struct Shgu64Smem {
-    alignas(16) uint8_t a[2][2][4096]; // [stage][token tile][32-block of hi|lo halves, qe_hl_off order]
-    alignas(16) uint8_t w[2][128][32]; // [stage][row: gate 0..63, up 64..127][32 int8]
-    _Float16 sc[QE_D / 32][128];       // [block][row]
+// gate rows + the same 64 up rows; S groups of four waves split K (their sums meet
+// in LDS), and wave w of a group takes token tile w & 1 and rows 32 (w >> 1) + 0..31
+// of both over the group's K.  Each 32-block of K, a group stages the 8 KB of
+// activations and 4 KB of Q8 rows in LDS once (double-buffered, one barrier per
+// block) and every wave reads its operands from there: each fetched byte feeds two
+// waves' MFMAs instead of one.  The Q8 block scales of the 128 rows sit in LDS for
+// the whole K, block-major, so the 32 rows a wave reads for one block are consecutive.
+template <int S> struct Shgu64Smem {
+    alignas(16) uint8_t a[S][2][2][4096]; // [group][stage][token tile][32-block of hi|lo halves, qe_hl_off order]
+    alignas(16) uint8_t w[S][2][128][32]; // [group][stage][row: gate 0..63, up 64..127][32 int8]
+    _Float16 sc[QE_D / 32][128];          // [block][row]
 };
-QE_DEV void shgu_tile64(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *hhl, int mp, int jg, Shgu64Smem &sm) {
+template <int S>
+QE_DEV void shgu_tile64(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *hhl, int mp, int jg, Shgu64Smem<S> &sm) {
     constexpr uint32_t RB = QE_SH_GU_ROW_BYTES;
-    constexpr int NB = QE_D / 32;
-    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, c = lane & 31, kh = lane >> 5;
-    const int mt32 = (T + 31) / 32, j0 = jg * 64;
+    constexpr int NB = QE_D / 32 / S; // blocks per group
+    const int tid = threadIdx.x & 255, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), lane = tid & 63, wv = tid >> 6,
+              c = lane & 31, kh = lane >> 5;
+    const int mt32 = (T + 31) / 32, j0 = jg * 64, kb0 = grp * NB;
     const __amdgpu_buffer_rsrc_t ra =
         __builtin_amdgcn_make_buffer_rsrc((void *)xhl, (short)0, mt32 * 32 * QE_D * 4, 0x00020000);
     const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc((void *)W, (short)0, (int)QE_SH_GU_BYTES, 0x00020000);
     auto row_off = [&](int r) -> uint32_t { return (uint32_t)((r < 64 ? 0 : QE_FF_SH - 64) + j0 + r) * RB; };
-    // block scales of the 128 rows: thread (row tid / 2, half tid & 1) brings 32 of them
+    // block scales of the 128 rows: thread (row tid / 2, half tid & 1) brings its half of the group's NB
     {
         const int r = tid >> 1, h = tid & 1;
-        qe_u32x4 s[4];
+        qe_u32x4 s[NB / 16];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s[i] = sh_ld(rw, row_off(r) + QE_D + 64 * h + 16 * i);
+        for (int i = 0; i < NB / 16; ++i) s[i] = sh_ld(rw, row_off(r) + QE_D + 2 * kb0 + NB * h + 16 * i);
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < NB / 16; ++i)
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const uint32_t v = s[i][e >> 1];
-                sm.sc[32 * h + 8 * i + e][r] = __builtin_bit_cast(_Float16, (uint16_t)((e & 1) ? v >> 16 : v & 0xffffu));
+                sm.sc[kb0 + NB / 2 * h + 8 * i + e][r] =
+                    __builtin_bit_cast(_Float16, (uint16_t)((e & 1) ? v >> 16 : v & 0xffffu));
             }
     }
     // staging roles: chunks tid, tid + 256 (activations of token tile 0, 1), tid + 512 (rows)
@@ -905,38 +935,63 @@ QE_DEV void shgu_tile64(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
         const int mt = 2 * mp + s < mt32 ? 2 * mp + s : mt32 - 1; // a tile past T reads the last one; never stored
-        a_src[s] = (uint32_t)mt * NB * 4096 + 16 * tid;
+        a_src[s] = (uint32_t)(mt * (QE_D / 32) + kb0) * 4096 + 16 * tid;
     }
     const int wr = tid >> 1, wh = tid & 1;
-    const uint32_t w_src = row_off(wr) + 16 * wh;
-    qe_u32x4 st[3];
-    auto fetch = [&](int b) {
-        st[0] = sh_ld(ra, a_src[0] + 4096 * b);
-        st[1] = sh_ld(ra, a_src[1] + 4096 * b);
-        st[2] = sh_ld(rw, w_src + 32 * b);
+    const uint32_t w_src = row_off(wr) + 32 * kb0 + 16 * wh;
+    qe_u32x4 st[2][3];
+    auto fetch = [&](int b, qe_u32x4 (&v)[3]) {
+        v[0] = sh_ld(ra, a_src[0] + 4096 * b);
+        v[1] = sh_ld(ra, a_src[1] + 4096 * b);
+        v[2] = sh_ld(rw, w_src + 32 * b);
     };
-    auto put = [&](int s) {
-        *(qe_u32x4 *)&sm.a[s][0][16 * tid] = st[0];
-        *(qe_u32x4 *)&sm.a[s][1][16 * tid] = st[1];
-        *(qe_u32x4 *)&sm.w[s][wr][16 * wh] = st[2];
+    auto put = [&](int s, const qe_u32x4 (&v)[3]) {
+        *(qe_u32x4 *)&sm.a[grp][s][0][16 * tid] = v[0];
+        *(qe_u32x4 *)&sm.a[grp][s][1][16 * tid] = v[1];
+        *(qe_u32x4 *)&sm.w[grp][s][wr][16 * wh] = v[2];
     };
-    fetch(0);
-    put(0);
+    fetch(0, st[0]);
+    put(0, st[0]);
+    fetch(1, st[1]);
     __syncthreads();
     const int ms = wv & 1, rg = 32 * (wv >> 1) + c, ru = 64 + rg;
     qe_float16v ag = {}, au = {};
-#pragma unroll 2
-    for (int b = 0; b < NB; ++b) {
-        const int s = b & 1;
-        if (b + 1 < NB) fetch(b + 1);
+    // block b from stage s; block b + 2 is fetched, b + 1 put into the other stage
+    auto block = [&](int b, int s) {
+        fetch(b + 2 < NB ? b + 2 : NB - 1, st[s]);
+        __builtin_amdgcn_sched_barrier(0);
         qe_u32x4 a[4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) a[q] = *(const qe_u32x4 *)&sm.a[s][ms][1024 * q + 16 * lane];
-        const qe_u32x4 wg = *(const qe_u32x4 *)&sm.w[s][rg][16 * kh], wu = *(const qe_u32x4 *)&sm.w[s][ru][16 * kh];
-        sh_block(a, wg, (float)sm.sc[b][rg], ag);
-        sh_block(a, wu, (float)sm.sc[b][ru], au);
-        if (b + 1 < NB) put(s ^ 1); // stage s ^ 1 was last read in block b - 1, before the barrier
+        for (int q = 0; q < 4; ++q) a[q] = *(const qe_u32x4 *)&sm.a[grp][s][ms][1024 * q + 16 * lane];
+        const qe_u32x4 wg = *(const qe_u32x4 *)&sm.w[grp][s][rg][16 * kh], wu = *(const qe_u32x4 *)&sm.w[grp][s][ru][16 * kh];
+        sh_block(a, wg, (float)sm.sc[kb0 + b][rg], ag);
+        sh_block(a, wu, (float)sm.sc[kb0 + b][ru], au);
+        put(s ^ 1, st[s ^ 1]); // stage s ^ 1 was last read in block b - 1, before the barrier
         __syncthreads();
+    };
+#pragma unroll 1
+    for (int b = 0; b < NB; b += 2) {
+        block(b, 0);
+        block(b + 1, 1);
+    }
+    static_assert(S == 1 || S == 2, "one group, or two whose sums meet");
+    if constexpr (S == 2) { // the second group's sums through the activation stages
+        float *red = (float *)&sm.a[0][0][0][0] + wv * 32 * 64 + lane;
+        static_assert(4 * 32 * 64 * 4 <= sizeof sm.a, "sums fit the stages");
+        if (grp == 1) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                red[64 * i] = ag[i];
+                red[64 * (16 + i)] = au[i];
+            }
+        }
+        __syncthreads();
+        if (grp == 1) return;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            ag[i] = ag[i] + red[64 * i];
+            au[i] = au[i] + red[64 * (16 + i)];
+        }
     }
     const int m0 = 64 * mp + 32 * ms, j = j0 + 32 * (wv >> 1) + c;
 #pragma unroll
@@ -952,11 +1007,12 @@ QE_DEV void shgu_tile64(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *
     }
 }
 // workgroup b on XCD b % 8: the 8 row groups of one 64-token pair back to back there
-__global__ __launch_bounds__(256) void k_shgu(const _Float16 *xhl, int T, const uint8_t *Wg, _Float16 *hhl) {
-    __shared__ Shgu64Smem sm;
+template <int S>
+__global__ __launch_bounds__(256 * S, 4) void k_shgu(const _Float16 *xhl, int T, const uint8_t *Wg, _Float16 *hhl) {
+    __shared__ Shgu64Smem<S> sm;
     const int x = blockIdx.x & 7, k = blockIdx.x >> 3, mp = 8 * (k / 8) + x;
     if (mp >= (T + 63) / 64) return;
-    shgu_tile64(xhl, T, Wg, hhl, mp, k % 8, sm);
+    shgu_tile64<S>(xhl, T, Wg, hhl, mp, k % 8, sm);
 }
 
 // Shared down, 64 tokens x 128 output rows per workgroup: wave w takes token
@@ -1341,12 +1397,25 @@ __global__ __launch_bounds__(256, 4) void k_expert_gudn(GemmTileArgs gu, GemmTil
 }
 
 hipError_t qe_launch_router_shgu(const QeLayerPtrs &L, const QeScratch &S, int T, hipStream_t st) {
-    const int nr = RS_NT * ((T + 63) / 64) * RT_SPLIT, ns = 8 * RS_JT * (((T + 31) / 32 + 7) / 8);
+    const int nz = qe_router_splits(T);
     if (T >= QE_RS_SPLIT_T) {
-        k_router<<<nr, 256, 0, st>>>(S.xn, T, L.router, S.rpart);
-        k_shgu<<<64 * (((T + 63) / 64 + 7) / 8), 256, 0, st>>>(S.xhl, T, L.sh_gu, (_Float16 *)S.shgu);
-    } else {
-        k_router_shgu<<<nr + ns, 256, 0, st>>>(S.xn, S.xhl, T, L.router, L.sh_gu, S.rpart, (_Float16 *)S.shgu);
+        const int grid = 16 * (((T + 63) / 64 * nz + 7) / 8);
+        switch (nz) {
+        case 4: k_router<4><<<grid, 256, 0, st>>>(S.xn, T, L.router, S.rpart); break;
+        default: k_router<3><<<grid, 256, 0, st>>>(S.xn, T, L.router, S.rpart); break;
+        }
+        const int gs = 64 * (((T + 63) / 64 + 7) / 8);
+        // below 4096 tokens the 64-token tiles alone leave CUs idle: two K groups per
+        // tile (1999 tokens: 48 -> 35 us; at 8192 one group, four workgroups per CU)
+        if (T < 4096) k_shgu<2><<<gs, 512, 0, st>>>(S.xhl, T, L.sh_gu, (_Float16 *)S.shgu);
+        else k_shgu<1><<<gs, 256, 0, st>>>(S.xhl, T, L.sh_gu, (_Float16 *)S.shgu);
+    } else { // XCD 0 has the most tiles of either kind
+        const int grid = 8 * (rs_router_per_xcd(T, nz, 0) + rs_shgu_per_xcd(T, 0));
+        const auto go = [&](auto kern) {
+            kern<<<grid, 512, 0, st>>>(S.xn, S.xhl, T, L.router, L.sh_gu, S.rpart, (_Float16 *)S.shgu);
+        };
+        if (nz == 16) go(k_router_shgu<2>);
+        else go(k_router_shgu<1>);
     }
     return hipGetLastError();
 }
