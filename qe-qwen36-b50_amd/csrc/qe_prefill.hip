@@ -120,7 +120,7 @@ QE_DEV void transpose_rows4(uint32_t d[4]) {
     d[0] = u.x; d[1] = u.y; d[2] = v.x; d[3] = v.y;
 }
 
-// LDS of one (NC, NT) tile, in bytes from the start of ExpertSmem::raw:
+// LDS of a big item's tile, in bytes from the start of ExpertSmem::raw:
 //   weight scales of the workgroup's rows, whole K: fp16 [block][wave][n][group];
 //   two stages of the item's activations for one quad (4 blocks): [pair][128 bytes],
 //     the 16-byte chunk q of pair m stored at chunk q ^ (m / 2 % 8) -- the sixteen
@@ -129,70 +129,49 @@ QE_DEV void transpose_rows4(uint32_t d[4]) {
 //   two stages of their block scales: fp32 [block of the quad][pair].
 // Stages of a quad rather than a turn keep a big item's workgroup at 34 KB, so
 // that four fit a CU.
-constexpr int qe_cmax(int a, int b) { return a > b ? a : b; }
-template <bool GU, int NC, int NT> struct TileLds {
-    static constexpr int NB = (GU ? QE_D : QE_FF_EXP) / 32;
-    static constexpr int DW = 0, DW_SZ = NB * 4 * 16 * NC * 2;
-    static constexpr int EPI = !GU ? 0
-                               : NC == 1 ? (2 * 16 * 16 * 4 + 2 * 16 * 4 + 16 * 32 + 2 * 16 * 4) * NT
-                                         : 4 * QE_MFMA_MC * 4 + 16 * NT * (64 + 8 + 8);
-    static constexpr int ACT = DW + DW_SZ, ACT_SZ = qe_cmax(16 * NT * 128, EPI);
+struct TileLds {
+    static constexpr int NT = QE_MFMA_MC / 16, NB = QE_D / 32;
+    static constexpr int DW = 0, DW_SZ = NB * 4 * 16 * 2 * 2;
+    static constexpr int EPI = 4 * QE_MFMA_MC * 4 + 16 * NT * (64 + 8 + 8);
+    static constexpr int ACT = DW + DW_SZ, ACT_SZ = 16 * NT * 128;
     static constexpr int XS = ACT + 2 * ACT_SZ, XS_SZ = 4 * 16 * NT * 4;
     static constexpr int SIZE = XS + 2 * XS_SZ;
+    static_assert(EPI <= ACT_SZ, "the epilogue fits one stage");
 };
-template <bool GU> struct ExpertSmem {
-    static constexpr int SIZE = qe_cmax(TileLds<GU, 2, 4>::SIZE, qe_cmax(TileLds<GU, 2, 2>::SIZE, TileLds<GU, 2, 1>::SIZE));
-    static_assert(TileLds<GU, 1, 2>::SIZE <= SIZE, "the one-matrix gate/up waves fit as well");
-    alignas(16) uint8_t raw[SIZE];
+struct ExpertSmem {
+    alignas(16) uint8_t raw[TileLds::SIZE];
     int pair[QE_MFMA_MC];
 };
 
-// Wave = NC column groups of 16 weight rows x NT 16-pair tiles (NC MFMAs per
-// block and tile; each weight decoded once per item).
-// Row groups yb of a workgroup (4 waves):
-//   gate/up, NC = 4: h rows 32 (4 yb + wave) + 0..31; groups gate, gate+16, up, up+16;
-//   gate/up, NC = 2: h rows 16 (4 yb + wave) + 0..15; groups gate, up -- a 32-block
-//            of h spans the wave pair (2w, 2w+1), which meets in LDS for its maximum;
-//   gate/up, NC = 1: h rows 32 yb + 16 (wave % 2) + 0..15 of the gate (waves 0, 1) or
-//            up (waves 2, 3) matrix -- half the rows of NC = 2 per workgroup, each
-//            output's K order unchanged; the up waves hand their dots to the gate
-//            waves through LDS;
-//   down:    output rows 64 NC yb + 16 NC wave + 16 c + 0..15.
-template <bool GU, int NC, int NT>
-__device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it, const int yb, ExpertSmem<GU> &sm) {
-    static_assert(NC == 2 || NC == 4 || (GU && NC == 1), "one (gate/up), two or four column groups per wave");
-    static_assert(16 * NT <= QE_MFMA_MC, "tiles of the item");
-    constexpr int KD = GU ? QE_D : QE_FF_EXP;  // reduction length
-    constexpr int NB = KD / 32;                // K blocks
+// Gate/up of a big item (33..64 pairs): wave = NC = 2 column groups of 16 weight rows
+// (gate, up) x NT = 4 16-pair tiles (NC MFMAs per block and tile; each weight decoded
+// once per item).  Workgroup yb (4 waves): h rows 16 (4 yb + wave) + 0..15; a 32-block
+// of h spans the wave pair (2w, 2w+1), which meets in LDS for its maximum.
+__device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it, const int yb, ExpertSmem &sm) {
+    constexpr int NC = 2, NT = TileLds::NT;
+    constexpr int KD = QE_D, NB = TileLds::NB; // reduction length, K blocks
     constexpr int NCH = NB / 8;                // turns (two quads each)
-    constexpr uint32_t RB = GU ? QE_GU_ROW_BYTES : QE_DN_ROW_BYTES;
+    constexpr uint32_t RB = QE_GU_ROW_BYTES;
     auto &s_pair = sm.pair;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, n = lane & 15, g = lane >> 4;
-    auto row_of = [&](int w, int c, int nn) -> int {
-        if constexpr (!GU) return yb * (64 * NC) + w * (16 * NC) + 16 * c + nn;
-        else if constexpr (NC == 4) return (c < 2 ? 0 : QE_FF_EXP) + (yb * 4 + w) * 32 + 16 * (c & 1) + nn;
-        else if constexpr (NC == 2) return (c == 0 ? 0 : QE_FF_EXP) + (yb * 4 + w) * 16 + nn;
-        else return (w < 2 ? 0 : QE_FF_EXP) + (yb * 2 + (w & 1)) * 16 + nn;
-    };
-    const uint8_t *ebase = a.arena + (size_t)it.x * QE_EXPERT_BYTES + (GU ? 0 : QE_EXPERT_DOWN_OFF);
+    auto row_of = [&](int w, int c, int nn) -> int { return (c == 0 ? 0 : QE_FF_EXP) + (yb * 4 + w) * 16 + nn; };
+    const uint8_t *ebase = a.arena + (size_t)it.x * QE_EXPERT_BYTES;
     // Buffer loads: a range-checked resource per operand (reads past the end
     // return 0), uniform per-turn offsets in SGPRs, per-lane offsets fixed.
-    const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-        (void *)ebase, (short)0, (int)(GU ? QE_EXPERT_DOWN_OFF : QE_EXPERT_BYTES - QE_EXPERT_DOWN_OFF), 0x00020000);
+    const __amdgpu_buffer_rsrc_t wr =
+        __builtin_amdgcn_make_buffer_rsrc((void *)ebase, (short)0, (int)QE_EXPERT_DOWN_OFF, 0x00020000);
     const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void *)a.aq, (short)0, a.a_bytes, 0x00020000);
     auto ld128 = [](__amdgpu_buffer_rsrc_t r, uint32_t vo, int so) {
         const qe_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0);
         return make_uint4(v.x, v.y, v.z, v.w);
     };
-    using LY = TileLds<GU, NC, NT>;
+    using LY = TileLds;
     uint8_t *const lds = sm.raw;
 
-    int rowc[NC];
     uint32_t boff[NC]; // byte offset of block g of the lane's row, per column group
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        rowc[c] = row_of(wv, c, n);
-        boff[c] = (uint32_t)rowc[c] * RB + 16 * g;
+        boff[c] = (uint32_t)row_of(wv, c, n) * RB + 16 * g;
     }
     // Ring: quad slot qs of turn ch holds blocks 8 ch + 4 qs .. +3; refills wrap
     // to turn (ch + 1) % NCH.
@@ -302,13 +281,7 @@ __device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it
             }
             {
                 uint32_t dep;
-                if constexpr (NC == 4)
-                    asm volatile("v_mov_b32 %0, 0" : "=v"(dep)
-                                 : "v"(cw[0][0]), "v"(cw[1][0]), "v"(cw[2][0]), "v"(cw[3][0]));
-                else if constexpr (NC == 2)
-                    asm volatile("v_mov_b32 %0, 0" : "=v"(dep) : "v"(cw[0][0]), "v"(cw[1][0]));
-                else
-                    asm volatile("v_mov_b32 %0, 0" : "=v"(dep) : "v"(cw[0][0]));
+                asm volatile("v_mov_b32 %0, 0" : "=v"(dep) : "v"(cw[0][0]), "v"(cw[1][0]));
                 load_q(nx, qs, dep);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -389,181 +362,277 @@ __device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it
     // the last quad (odd) read stage 1: the epilogue works in stage 0
 
     // lane holds rows 16 t + 4 g + i, column n of each group
-    if constexpr (GU && NC == 4) {
-        const int jb = yb * 4 + wv; // 32-block of h
+    // h rows 16 (4 yb + wv) + n: half (wv & 1) of 32-block jb
+    const int jb = yb * 2 + (wv >> 1), half = wv & 1;
+    // each wave's |h| maximum per pair, in the activation stage the last turn
+    // did not read (stage 0: its last reader passed the barrier that ended quad 2 NCH - 2)
+    float(*amax)[QE_MFMA_MC] = (float(*)[QE_MFMA_MC])(sm.raw + LY::ACT);
+    static_assert(4 * QE_MFMA_MC * 4 <= LY::ACT_SZ, "maxima fit one stage");
+    float h[NT][4], m[NT][4];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const float h0 = silu_mul(acc[0][t][i], acc[2][t][i]);
-                const float h1 = silu_mul(acc[1][t][i], acc[3][t][i]);
-                float m = fmaxf(fabsf(h0), fabsf(h1));
-                m = max16(m);
-                float d;
-                const float id = quant_scale_inv(m, d);
-                const int p = s_pair[16 * t + 4 * g + i];
-                if (p >= 0) {
-                    int8_t *hrow = a.hq + (size_t)p * QE_FF_EXP + (jb >> 1) * 64 + (n >> 2) * 16 + (jb & 1) * 8 + (n & 3);
-                    hrow[0] = quant_one(h0, id);
-                    hrow[4] = quant_one(h1, id);
-                    if (n == 0) a.hs[(size_t)p * (QE_FF_EXP / 32) + jb] = d;
-                }
+        for (int i = 0; i < 4; ++i) {
+            h[t][i] = silu_mul(acc[0][t][i], acc[1][t][i]);
+            m[t][i] = max16_abs(h[t][i]);
+            if (n == 0) amax[wv][16 * t + 4 * g + i] = m[t][i];
+        }
+    __syncthreads();
+    // The workgroup's h of a pair is the 64 contiguous bytes [64 yb, 64 yb + 64) of its
+    // row in the operand layout (blocks 2 yb, 2 yb + 1), and its two block scales are
+    // adjacent: both are assembled in LDS (after the maxima, in the same free stage)
+    // and stored 16 bytes per thread, instead of one byte per lane and value.
+    uint8_t *htile = sm.raw + LY::ACT + 4 * QE_MFMA_MC * 4; // [16 NT][64]
+    float *stile = (float *)(htile + 16 * NT * 64);                                  // [16 NT][2]
+    float *itile = stile + 16 * NT * 2;                                              // [2][16 NT] inverses
+    static_assert(4 * QE_MFMA_MC * 4 + 16 * NT * (64 + 8 + 8) <= LY::ACT_SZ, "h tile fits the free stage");
+    if (tid < 2 * 16 * NT) { // block (jb % 2 = wave pair) scale and its inverse, once per pair
+        const int pr = tid / (16 * NT), mi = tid % (16 * NT);
+        float d;
+        itile[tid] = quant_scale_inv(fmaxf(amax[2 * pr][mi], amax[2 * pr + 1][mi]), d);
+        stile[mi * 2 + pr] = d;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const float4 id4 = *(const float4 *)(itile + (wv >> 1) * 16 * NT + 16 * t + 4 * g);
+        const float id[4] = {id4.x, id4.y, id4.z, id4.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int mi = 16 * t + 4 * g + i;
+            htile[mi * 64 + (n >> 2) * 16 + (jb & 1) * 8 + (n & 3) + 4 * half] = (uint8_t)quant_one(h[t][i], id[i]);
+        }
+    }
+    __syncthreads();
+    {   // thread (pair tid / 4, 16-byte part tid % 4)
+        const int mi = tid >> 2, q = tid & 3;
+        const int p = mi < 16 * NT ? s_pair[mi] : -1;
+        if (p >= 0) {
+            int8_t *hp = a.hq + (size_t)p * QE_FF_EXP + (jb >> 1) * 64 + 16 * q;
+            float *sp = a.hs + (size_t)p * (QE_FF_EXP / 32) + 2 * (jb >> 1);
+            if (a.item_done) { // fused launch: written through for its down workgroups
+                st_sc1(hp, *(const uint4 *)(htile + mi * 64 + 16 * q));
+                if (q == 0) st_sc1(sp, *(const uint2 *)(stile + mi * 2));
+            } else {
+                *(uint4 *)hp = *(const uint4 *)(htile + mi * 64 + 16 * q);
+                if (q == 0) *(float2 *)sp = *(const float2 *)(stile + mi * 2);
             }
         }
-    } else if constexpr (GU && NC == 1) {
-        // 32-block yb of h: rows 16 rs + n, rs = wv % 2, from gate wave rs and up wave
-        // 2 + rs.  All of it goes through stage 0, which the last quad did not read.
-        uint8_t *fs = sm.raw + LY::ACT;
-        float *utile = (float *)fs;                              // [2][16 NT pairs][16] the up dots
-        float *amax = utile + 2 * 16 * NT * 16;                  // [2][16 NT] |h| maxima per half
-        uint8_t *htile = (uint8_t *)(amax + 2 * 16 * NT);         // [16 NT][32] int8 h, operand order
-        float *stile = (float *)(htile + 16 * NT * 32);          // [16 NT] block scales
-        float *itile = stile + 16 * NT;                          // [16 NT] their inverses
-        static_assert((2 * 16 * 16 * 4 + 2 * 16 * 4 + 16 * 32 + 2 * 16 * 4) * NT <= LY::ACT_SZ,
-                      "the epilogue fits the free stage");
-        const int rs = wv & 1;
-        if (wv >= 2) {
+    }
+}
+
+// Gate/up of a small item (<= 16 NT pairs): workgroup = 32 h rows, waves 0, 1 the
+// gate rows 32 yb + 16 (wave % 2) + 0..15, waves 2, 3 the up rows; the up waves hand
+// their dots to the gate waves through LDS.  These items hold few pairs, so they
+// stream weights for little arithmetic and what counts is bytes in flight: the
+// block scales of rows and pairs are staged in LDS once, and then each wave streams
+// its codes (a ring of four quads) and its activations (straight from L1/L2 in the
+// operand layout, RA quads ahead) with no barrier until the epilogue.  (Activations
+// staged through LDS a quad ahead, one barrier a quad, tied every quad to an L2 round
+// trip: k_expert_gu at 12 tokens, 82 experts, 31.9 us against 27.4; the fused launch
+// at 100 tokens 127 against 123.)  Arithmetic and K order as expert_tile.
+template <int NT> struct GuSmallLds {
+    static constexpr int NB = QE_D / 32;
+    static constexpr int DW = 0, XS = DW + NB * 64 * 2; // fp16 [block][wave][n]; fp32 [block][pair]
+    static constexpr int EPI = XS + NB * 16 * NT * 4;
+    static constexpr int SIZE = EPI + (2 * 16 * 16 * 4 + 2 * 16 * 4 + 16 * 32 + 2 * 16 * 4) * NT;
+};
+template <int NT>
+__device__ __forceinline__ void gu_small(const GemmTileArgs &a, const int4 it, const int yb, ExpertSmem &sm) {
+    using LY = GuSmallLds<NT>;
+    static_assert(LY::SIZE <= TileLds::SIZE, "the small items' tile fits as well");
+    constexpr int NB = LY::NB, NQ = NB / 4, RC = 4, RA = 4 / NT;
+    constexpr uint32_t RB = QE_GU_ROW_BYTES;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, n = lane & 15, g = lane >> 4;
+    auto &s_pair = sm.pair;
+    uint8_t *const lds = sm.raw;
+    auto row_of = [&](int w, int nn) -> int { return (w < 2 ? 0 : QE_FF_EXP) + (yb * 2 + (w & 1)) * 16 + nn; };
+    const uint8_t *ebase = a.arena + (size_t)it.x * QE_EXPERT_BYTES;
+    const __amdgpu_buffer_rsrc_t wr =
+        __builtin_amdgcn_make_buffer_rsrc((void *)ebase, (short)0, (int)QE_EXPERT_DOWN_OFF, 0x00020000);
+    const __amdgpu_buffer_rsrc_t ar = __builtin_amdgcn_make_buffer_rsrc((void *)a.aq, (short)0, a.a_bytes, 0x00020000);
+    const uint32_t boff = (uint32_t)row_of(wv, n) * RB + 16 * g; // block g of the lane's row
+    qe_u32x4 rq[RC];          // raw codes: lane (n, g) holds block 4 Q + g of its row
+    qe_u32x4 ra[RA][2][NT];   // activations: block pair jp of the quad, tile t
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+    for (int q = 0; q < RC; ++q) rq[q] = __builtin_amdgcn_raw_buffer_load_b128(wr, boff, 64 * q, 0);
+    // thread (row tid / 4, quarter tid % 4): 16 of the row's 64 weight scales
+    qe_u32x4 dwv[2];
+    {
+        const uint32_t so = (uint32_t)row_of(tid >> 6, (tid >> 2) & 15) * RB + QE_D / 2 + 32 * (tid & 3);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) utile[(rs * 16 * NT + 16 * t + 4 * g + i) * 16 + n] = acc[0][t][i];
+        for (int i = 0; i < 2; ++i) dwv[i] = __builtin_amdgcn_raw_buffer_load_b128(wr, so, 16 * i, 0);
+    }
+    if (tid < QE_MFMA_MC) s_pair[tid] = tid < it.z ? a.pairs[it.y + tid] : -1;
+    __syncthreads();
+    uint32_t aoff[NT]; // the lane's activation row (padding pairs read pair 0's; their scales are 0)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int p = s_pair[16 * t + n];
+        aoff[t] = (uint32_t)((p < 0 ? s_pair[0] : p) / QE_K_USED) * QE_D + 16 * g;
+    }
+    auto load_a = [&](int qq, int slot) {
+#pragma unroll
+        for (int jp = 0; jp < 2; ++jp)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) ra[slot][jp][t] = __builtin_amdgcn_raw_buffer_load_b128(ar, aoff[t], 128 * qq + 64 * jp, 0);
+    };
+#pragma unroll
+    for (int q = 0; q < RA; ++q) load_a(q, q);
+    {   // pair scales: thread (pair tid % (16 NT), quads q0, q0 + 16 / NT, ..)
+        const int m = tid & (16 * NT - 1), q0 = tid / (16 * NT), p = s_pair[m];
+        const float4 *src = (const float4 *)(a.as + (size_t)((p < 0 ? s_pair[0] : p) / QE_K_USED) * NB);
+        float *xs = (float *)(lds + LY::XS) + m;
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+            const int q = q0 + 16 / NT * k;
+            float4 v = src[q];
+            if (p < 0) v = make_float4(0.f, 0.f, 0.f, 0.f);
+            xs[(4 * q + 0) * 16 * NT] = v.x;
+            xs[(4 * q + 1) * 16 * NT] = v.y;
+            xs[(4 * q + 2) * 16 * NT] = v.z;
+            xs[(4 * q + 3) * 16 * NT] = v.w;
         }
-        __syncthreads();
-        float h[NT][4], m[NT][4];
-        if (wv < 2) {
+        uint16_t *dwl = (uint16_t *)(lds + LY::DW) + 16 * (tid & 3) * 64 + (tid >> 2);
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int mi = 16 * t + 4 * g + i;
-                    h[t][i] = silu_mul(acc[0][t][i], utile[(rs * 16 * NT + mi) * 16 + n]);
-                    m[t][i] = max16_abs(h[t][i]);
-                    if (n == 0) amax[rs * 16 * NT + mi] = m[t][i];
-                }
+            for (int j = 0; j < 8; ++j) dwl[(8 * i + j) * 64] = (uint16_t)(dwv[i][j >> 1] >> (16 * (j & 1)));
+    }
+    __syncthreads();
+
+    float acc[NT][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[t][i] = 0.f;
+    // quad qq from ring slots sc, sa; then slot sc takes quad qq + RC, sa quad qq + RA
+    auto quad = [&](int qq, int sc, int sa, bool more_c, bool more_a) {
+        uint32_t cw[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) asm volatile("v_mov_b32 %0, %1" : "=v"(cw[k]) : "v"(rq[sc][k]));
+        transpose_rows4(cw);
+        if (more_c) {
+            uint32_t dep;
+            asm volatile("v_mov_b32 %0, 0" : "=v"(dep) : "v"(cw[0]));
+            rq[sc] = __builtin_amdgcn_raw_buffer_load_b128(wr, boff + dep, 64 * (qq + RC), 0);
+            __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
-        if (tid < 16 * NT) { // the block's scale and its inverse, once per pair
-            float d;
-            itile[tid] = quant_scale_inv(fmaxf(amax[tid], amax[16 * NT + tid]), d);
-            stile[tid] = d;
-        }
-        __syncthreads();
-        if (wv < 2) {
-            // element 16 rs + n of the block: byte (n / 4) * 16 + (yb % 2) * 8 + n % 4 + 4 rs
-            // of the pair's 64-byte run (yb / 2) of h (the layout of the NC = 2 path);
-            // htile keeps this block's 8-byte groups n / 4 contiguous
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
+        for (int j = 0; j < 4; ++j) {
+            const int b = 4 * qq + j, jp = j >> 1;
+            uint32_t lo, hi;
+            nl4_decode_dword<true>(cw[j], lo, hi);
+            const long bv = (long)(((uint64_t)hi << 32) | lo);
+            float dwf = (float)*(const _Float16 *)(lds + LY::DW + (b * 64 + wv * 16 + n) * 2), cng = dwf * -QE_I2F_MAGIC;
+            asm volatile("" : "+v"(dwf), "+v"(cng));
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int mi = 16 * t + 4 * g + i;
-                    htile[mi * 32 + (n >> 2) * 8 + (n & 3) + 4 * rs] = (uint8_t)quant_one(h[t][i], itile[mi]);
-                }
-        }
-        __syncthreads();
-        {   // thread (pair tid / 4, 8-byte group tid % 4)
-            const int mi = tid >> 2, q = tid & 3;
-            const int p = mi < 16 * NT ? s_pair[mi] : -1;
-            if (p >= 0) {
-                int8_t *hp = a.hq + (size_t)p * QE_FF_EXP + (yb >> 1) * 64 + 16 * q + 8 * (yb & 1);
-                float *sp = a.hs + (size_t)p * (QE_FF_EXP / 32) + yb;
-                if (a.item_done) { // fused launch: written through for its down workgroups
-                    st_sc1(hp, *(const uint2 *)(htile + mi * 32 + 8 * q));
-                    if (q == 0) st_sc1(sp, stile[mi]);
-                } else {
-                    *(uint2 *)hp = *(const uint2 *)(htile + mi * 32 + 8 * q);
-                    if (q == 0) *sp = stile[mi];
-                }
+            for (int t = 0; t < NT; ++t) {
+                const qe_u32x4 v = ra[sa][jp][t];
+                const long av = (j & 1) ? (long)(((uint64_t)v.w << 32) | v.z) : (long)(((uint64_t)v.y << 32) | v.x);
+                typedef int i32x4 __attribute__((ext_vector_type(4)));
+                const i32x4 mag = {QE_I2F_MAGIC_BITS, QE_I2F_MAGIC_BITS, QE_I2F_MAGIC_BITS, QE_I2F_MAGIC_BITS};
+                const i32x4 P = __builtin_amdgcn_mfma_i32_16x16x32_i8(av, bv, mag, 0, 0, 0);
+                const float4 x4 = *(const float4 *)(lds + LY::XS + (b * 16 * NT + 16 * t + 4 * g) * 4);
+                acc[t][0] = fmaf(fmaf(__int_as_float(P[0]), dwf, cng), x4.x, acc[t][0]);
+                acc[t][1] = fmaf(fmaf(__int_as_float(P[1]), dwf, cng), x4.y, acc[t][1]);
+                acc[t][2] = fmaf(fmaf(__int_as_float(P[2]), dwf, cng), x4.z, acc[t][2]);
+                acc[t][3] = fmaf(fmaf(__int_as_float(P[3]), dwf, cng), x4.w, acc[t][3]);
             }
         }
-    } else if constexpr (GU) {
-        // h rows 16 (4 yb + wv) + n: half (wv & 1) of 32-block jb
-        const int jb = yb * 2 + (wv >> 1), half = wv & 1;
-        // each wave's |h| maximum per pair, in the activation stage the last turn
-        // did not read (stage 0: its last reader passed the barrier that ended quad 2 NCH - 2)
-        float(*amax)[QE_MFMA_MC] = (float(*)[QE_MFMA_MC])(sm.raw + LY::ACT);
-        static_assert(4 * QE_MFMA_MC * 4 <= LY::ACT_SZ, "maxima fit one stage");
-        float h[NT][4], m[NT][4];
+        // scale now: left alone the compiler defers it, keeping every block product live
+#pragma unroll
+        for (int t = 0; t < NT; ++t) asm volatile("" : "+v"(acc[t][0]), "+v"(acc[t][1]), "+v"(acc[t][2]), "+v"(acc[t][3]));
+        if (more_a) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_a(qq + RA, sa);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+#pragma unroll 1
+    for (int q0 = 0; q0 + RC < NQ; q0 += RC) {
+#pragma unroll
+        for (int s = 0; s < RC; ++s) quad(q0 + s, s, s % RA, true, true);
+    }
+#pragma unroll
+    for (int s = 0; s < RC; ++s) quad(NQ - RC + s, s, s % RA, false, s + RA < RC);
+
+    // 32-block yb of h: rows 16 rs + n, rs = wv % 2, from gate wave rs and up wave
+    // 2 + rs
+    uint8_t *fs = lds + LY::EPI;
+    float *utile = (float *)fs;                              // [2][16 NT pairs][16] the up dots
+    float *amax = utile + 2 * 16 * NT * 16;                  // [2][16 NT] |h| maxima per half
+    uint8_t *htile = (uint8_t *)(amax + 2 * 16 * NT);         // [16 NT][32] int8 h, operand order
+    float *stile = (float *)(htile + 16 * NT * 32);          // [16 NT] block scales
+    float *itile = stile + 16 * NT;                          // [16 NT] their inverses
+    const int rs = wv & 1;
+    if (wv >= 2) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) utile[(rs * 16 * NT + 16 * t + 4 * g + i) * 16 + n] = acc[t][i];
+    }
+    __syncthreads();
+    float h[NT][4], m[NT][4];
+    if (wv < 2) {
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                h[t][i] = silu_mul(acc[0][t][i], acc[1][t][i]);
+                const int mi = 16 * t + 4 * g + i;
+                h[t][i] = silu_mul(acc[t][i], utile[(rs * 16 * NT + mi) * 16 + n]);
                 m[t][i] = max16_abs(h[t][i]);
-                if (n == 0) amax[wv][16 * t + 4 * g + i] = m[t][i];
+                if (n == 0) amax[rs * 16 * NT + mi] = m[t][i];
             }
-        __syncthreads();
-        // The workgroup's h of a pair is the 64 contiguous bytes [64 yb, 64 yb + 64) of its
-        // row in the operand layout (blocks 2 yb, 2 yb + 1), and its two block scales are
-        // adjacent: both are assembled in LDS (after the maxima, in the same free stage)
-        // and stored 16 bytes per thread, instead of one byte per lane and value.
-        uint8_t *htile = sm.raw + LY::ACT + 4 * QE_MFMA_MC * 4; // [16 NT][64]
-        float *stile = (float *)(htile + 16 * NT * 64);                                  // [16 NT][2]
-        float *itile = stile + 16 * NT * 2;                                              // [2][16 NT] inverses
-        static_assert(4 * QE_MFMA_MC * 4 + 16 * NT * (64 + 8 + 8) <= LY::ACT_SZ, "h tile fits the free stage");
-        if (tid < 2 * 16 * NT) { // block (jb % 2 = wave pair) scale and its inverse, once per pair
-            const int pr = tid / (16 * NT), mi = tid % (16 * NT);
-            float d;
-            itile[tid] = quant_scale_inv(fmaxf(amax[2 * pr][mi], amax[2 * pr + 1][mi]), d);
-            stile[mi * 2 + pr] = d;
-        }
-        __syncthreads();
+    }
+    __syncthreads();
+    if (tid < 16 * NT) { // the block's scale and its inverse, once per pair
+        float d;
+        itile[tid] = quant_scale_inv(fmaxf(amax[tid], amax[16 * NT + tid]), d);
+        stile[tid] = d;
+    }
+    __syncthreads();
+    if (wv < 2) {
+        // element 16 rs + n of the block: byte (n / 4) * 16 + (yb % 2) * 8 + n % 4 + 4 rs
+        // of the pair's 64-byte run (yb / 2) of h (as expert_tile);
+        // htile keeps this block's 8-byte groups n / 4 contiguous
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const float4 id4 = *(const float4 *)(itile + (wv >> 1) * 16 * NT + 16 * t + 4 * g);
-            const float id[4] = {id4.x, id4.y, id4.z, id4.w};
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int mi = 16 * t + 4 * g + i;
-                htile[mi * 64 + (n >> 2) * 16 + (jb & 1) * 8 + (n & 3) + 4 * half] = (uint8_t)quant_one(h[t][i], id[i]);
+                htile[mi * 32 + (n >> 2) * 8 + (n & 3) + 4 * rs] = (uint8_t)quant_one(h[t][i], itile[mi]);
             }
-        }
-        __syncthreads();
-        {   // thread (pair tid / 4, 16-byte part tid % 4)
-            const int mi = tid >> 2, q = tid & 3;
-            const int p = mi < 16 * NT ? s_pair[mi] : -1;
-            if (p >= 0) {
-                int8_t *hp = a.hq + (size_t)p * QE_FF_EXP + (jb >> 1) * 64 + 16 * q;
-                float *sp = a.hs + (size_t)p * (QE_FF_EXP / 32) + 2 * (jb >> 1);
-                if (a.item_done) { // fused launch: written through for its down workgroups
-                    st_sc1(hp, *(const uint4 *)(htile + mi * 64 + 16 * q));
-                    if (q == 0) st_sc1(sp, *(const uint2 *)(stile + mi * 2));
-                } else {
-                    *(uint4 *)hp = *(const uint4 *)(htile + mi * 64 + 16 * q);
-                    if (q == 0) *(float2 *)sp = *(const float2 *)(stile + mi * 2);
-                }
-            }
-        }
-    } else {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int p = s_pair[16 * t + 4 * g + i];
-                if (p < 0) continue;
-                const float w = a.wts[p];
-                float *yrow = a.yp + (size_t)p * QE_D;
-#pragma unroll
-                for (int c = 0; c < NC; ++c) yrow[rowc[c]] = w * acc[c][t][i];
+    }
+    __syncthreads();
+    {   // thread (pair tid / 4, 8-byte group tid % 4)
+        const int mi = tid >> 2, q = tid & 3;
+        const int p = mi < 16 * NT ? s_pair[mi] : -1;
+        if (p >= 0) {
+            int8_t *hp = a.hq + (size_t)p * QE_FF_EXP + (yb >> 1) * 64 + 16 * q + 8 * (yb & 1);
+            float *sp = a.hs + (size_t)p * (QE_FF_EXP / 32) + yb;
+            if (a.item_done) { // fused launch: written through for its down workgroups
+                st_sc1(hp, *(const uint2 *)(htile + mi * 32 + 8 * q));
+                if (q == 0) st_sc1(sp, stile[mi]);
+            } else {
+                *(uint2 *)hp = *(const uint2 *)(htile + mi * 32 + 8 * q);
+                if (q == 0) *sp = stile[mi];
             }
         }
     }
 }
 
 // Gate/up: big items (33..64 pairs, the first n_items[1]) run NT = 4, NC = 2
-// on 8 row groups of 64 h rows; the small ones after them NT = 2 or 1 on
-// NC = 1, 16 row groups of 32 h rows: twice the workgroups of half the life
-// (these items run last, after the big ones, and their workgroups had made the
-// launch's tail).  Workgroup b runs on XCD x = b % 8 (round-robin dispatch) and
+// on 8 row groups of 64 h rows; the small ones after them gu_small on
+// 16 row groups of 32 h rows: twice the workgroups of half the life (these items
+// run last, after the big ones, and their workgroups had made the launch's tail).  Workgroup b runs on XCD x = b % 8 (round-robin dispatch) and
 // takes the (b / 8)-th row group of that XCD's items x, x + 8, ..., the big
 // ones' first: all row groups of an item run on one XCD, so its activations
 // come from HBM once and from that XCD's L2 after.  (The odd row groups of a
 // big item as empty workgroups instead, interleaved with its real ones, left
 // half the CUs without work: the dispatcher deals an XCD's workgroups to its
 // CUs in turn.)
-template <bool GU> constexpr int expert_rg() { return GU ? QE_FF_EXP / 32 : QE_D / 128; }
-template <bool GU> QE_DEV void expert_unit(const GemmTileArgs &a, int b, ExpertSmem<GU> &sm) {
-    static_assert(GU, "the down items run dn_unit");
+QE_DEV void expert_unit(const GemmTileArgs &a, int b, ExpertSmem &sm) {
     const int x = b & 7, k = b >> 3, nbig = a.n_items[1];
     const int nbx = nbig > x ? (nbig - x + 7) >> 3 : 0; // big items on this XCD
     const bool big = k < 8 * nbx;
@@ -573,11 +642,11 @@ template <bool GU> QE_DEV void expert_unit(const GemmTileArgs &a, int b, ExpertS
     const int4 it = a.items[item];
     static_assert(QE_MFMA_MC == 64, "items of up to four 16-row tiles");
     if (big)
-        expert_tile<GU, 2, 4>(a, it, yb, sm);
+        expert_tile(a, it, yb, sm);
     else if (it.z > 16)
-        expert_tile<GU, 1, 2>(a, it, yb, sm);
+        gu_small<2>(a, it, yb, sm);
     else
-        expert_tile<GU, 1, 1>(a, it, yb, sm);
+        gu_small<1>(a, it, yb, sm);
     if (a.item_done) {
         // fused launch: every thread's h stores (sc1, written through) are acknowledged
         // before the item's count of finished gate/up workgroups goes up
@@ -589,12 +658,12 @@ template <bool GU> QE_DEV void expert_unit(const GemmTileArgs &a, int b, ExpertS
 // Workgroups over the items of np pairs: an upper bound of the item count
 // (items of more than QE_MFMA_MC / 2 pairs, plus at most one smaller item per
 // expert) rounded up to whole groups of 8 items, times the row groups.
-template <bool GU> constexpr int expert_max_wg(int np) {
-    return expert_rg<GU>() * (((np / (QE_MFMA_MC / 2 + 1) + 1 + QE_N_EXPERT) + 7) & ~7);
+constexpr int expert_max_wg(int np) {
+    return QE_FF_EXP / 32 * (((np / (QE_MFMA_MC / 2 + 1) + 1 + QE_N_EXPERT) + 7) & ~7);
 }
 __global__ __launch_bounds__(256, 4) void k_expert_gu(GemmTileArgs a) {
-    __shared__ ExpertSmem<true> sm;
-    expert_unit<true>(a, blockIdx.x, sm);
+    __shared__ ExpertSmem sm;
+    expert_unit(a, blockIdx.x, sm);
 }
 
 
@@ -1372,7 +1441,7 @@ __global__ __launch_bounds__(256, 2) void k_expert_dn(GemmTileArgs a, int nr, co
 __global__ __launch_bounds__(256, 4) void k_expert_gudn(GemmTileArgs gu, GemmTileArgs dn, int nshx,
                                                         const _Float16 *hhl, int T, const uint8_t *Wsd, float *sd) {
     __shared__ union {
-        ExpertSmem<true> g;
+        ExpertSmem g;
         DnSmem d;
         Shdn64Lds s;
     } sm;
@@ -1381,7 +1450,7 @@ __global__ __launch_bounds__(256, 4) void k_expert_gudn(GemmTileArgs gu, GemmTil
     const int nix = ni > x ? (ni - x + 7) >> 3 : 0, nbx = nb > x ? (nb - x + 7) >> 3 : 0; // items x, x + 8, ..
     const int gux = 8 * nbx + 16 * (nix - nbx);
     if (k < gux) {
-        expert_unit<true>(gu, b, sm.g);
+        expert_unit(gu, b, sm.g);
         return;
     }
     int r = k - gux;
@@ -1436,7 +1505,7 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
         g.item_done = S.item_done; g.err = S.err; g.err_val = S.err_val; g.spin_cap = S.spin_cap;
         g.wait_extra = S.wait_extra;
     } else {
-        k_expert_gu<<<expert_max_wg<true>(np), 256, 0, st>>>(g);
+        k_expert_gu<<<expert_max_wg(np), 256, 0, st>>>(g);
     }
     GemmTileArgs d = g;
     d.aq = S.hqp; d.a_bytes = np * QE_FF_EXP; d.as = S.hs; d.a_row_div = 1; d.yp = S.yp;
