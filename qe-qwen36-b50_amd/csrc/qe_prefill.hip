@@ -54,6 +54,7 @@ struct GemmTileArgs {
     int a_bytes;               // size of aq in bytes
     const float *as;           // their fp32 block scales
     int a_row_div;             // pair -> activation row: p / a_row_div (8 for tokens, 1 for pairs)
+    int direct;                // gate/up: small items take gu_small
     const int32_t *pairs;
     const int4 *items;         // (expert, first pair, count <= QE_MFMA_MC)
     const int32_t *n_items;
@@ -120,7 +121,78 @@ QE_DEV void transpose_rows4(uint32_t d[4]) {
     d[0] = u.x; d[1] = u.y; d[2] = v.x; d[3] = v.y;
 }
 
-// LDS of a big item's tile, in bytes from the start of ExpertSmem::raw:
+// Epilogue of the one-matrix waves (16 NT pairs, 32 h rows a workgroup): the up waves
+// hand their dots to the gate waves through `fs` (gu_epi_bytes<NT>() of LDS that no
+// wave reads any more), h is quantised per 32-block and stored.
+template <int NT> constexpr int gu_epi_bytes() { return (2 * 16 * 16 * 4 + 2 * 16 * 4 + 16 * 32 + 2 * 16 * 4) * NT; }
+template <int NT>
+QE_DEV void one_matrix_epilogue(const GemmTileArgs &a, const int yb, const int *s_pair, const float (&acc)[NT][4], uint8_t *fs) {
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, n = lane & 15, g = lane >> 4;
+    // 32-block yb of h: rows 16 rs + n, rs = wv % 2, from gate wave rs and up wave
+    // 2 + rs
+    float *utile = (float *)fs;                              // [2][16 NT pairs][16] the up dots
+    float *amax = utile + 2 * 16 * NT * 16;                  // [2][16 NT] |h| maxima per half
+    uint8_t *htile = (uint8_t *)(amax + 2 * 16 * NT);         // [16 NT][32] int8 h, operand order
+    float *stile = (float *)(htile + 16 * NT * 32);          // [16 NT] block scales
+    float *itile = stile + 16 * NT;                          // [16 NT] their inverses
+    const int rs = wv & 1;
+    if (wv >= 2) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) utile[(rs * 16 * NT + 16 * t + 4 * g + i) * 16 + n] = acc[t][i];
+    }
+    __syncthreads();
+    float h[NT][4], m[NT][4];
+    if (wv < 2) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int mi = 16 * t + 4 * g + i;
+                h[t][i] = silu_mul(acc[t][i], utile[(rs * 16 * NT + mi) * 16 + n]);
+                m[t][i] = max16_abs(h[t][i]);
+                if (n == 0) amax[rs * 16 * NT + mi] = m[t][i];
+            }
+    }
+    __syncthreads();
+    if (tid < 16 * NT) { // the block's scale and its inverse, once per pair
+        float d;
+        itile[tid] = quant_scale_inv(fmaxf(amax[tid], amax[16 * NT + tid]), d);
+        stile[tid] = d;
+    }
+    __syncthreads();
+    if (wv < 2) {
+        // element 16 rs + n of the block: byte (n / 4) * 16 + (yb % 2) * 8 + n % 4 + 4 rs
+        // of the pair's 64-byte run (yb / 2) of h (as expert_tile);
+        // htile keeps this block's 8-byte groups n / 4 contiguous
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int mi = 16 * t + 4 * g + i;
+                htile[mi * 32 + (n >> 2) * 8 + (n & 3) + 4 * rs] = (uint8_t)quant_one(h[t][i], itile[mi]);
+            }
+    }
+    __syncthreads();
+    {   // thread (pair tid / 4, 8-byte group tid % 4)
+        const int mi = tid >> 2, q = tid & 3;
+        const int p = mi < 16 * NT ? s_pair[mi] : -1;
+        if (p >= 0) {
+            int8_t *hp = a.hq + (size_t)p * QE_FF_EXP + (yb >> 1) * 64 + 16 * q + 8 * (yb & 1);
+            float *sp = a.hs + (size_t)p * (QE_FF_EXP / 32) + yb;
+            if (a.item_done) { // fused launch: written through for its down workgroups
+                st_sc1(hp, *(const uint2 *)(htile + mi * 32 + 8 * q));
+                if (q == 0) st_sc1(sp, stile[mi]);
+            } else {
+                *(uint2 *)hp = *(const uint2 *)(htile + mi * 32 + 8 * q);
+                if (q == 0) *sp = stile[mi];
+            }
+        }
+    }
+}
+
+// LDS of one (NC, NT) tile, in bytes from the start of ExpertSmem::raw:
 //   weight scales of the workgroup's rows, whole K: fp16 [block][wave][n][group];
 //   two stages of the item's activations for one quad (4 blocks): [pair][128 bytes],
 //     the 16-byte chunk q of pair m stored at chunk q ^ (m / 2 % 8) -- the sixteen
@@ -129,32 +201,42 @@ QE_DEV void transpose_rows4(uint32_t d[4]) {
 //   two stages of their block scales: fp32 [block of the quad][pair].
 // Stages of a quad rather than a turn keep a big item's workgroup at 34 KB, so
 // that four fit a CU.
-struct TileLds {
-    static constexpr int NT = QE_MFMA_MC / 16, NB = QE_D / 32;
-    static constexpr int DW = 0, DW_SZ = NB * 4 * 16 * 2 * 2;
-    static constexpr int EPI = 4 * QE_MFMA_MC * 4 + 16 * NT * (64 + 8 + 8);
-    static constexpr int ACT = DW + DW_SZ, ACT_SZ = 16 * NT * 128;
+template <int NC, int NT> struct TileLds {
+    static constexpr int NB = QE_D / 32;
+    static constexpr int DW = 0, DW_SZ = NB * 4 * 16 * NC * 2;
+    static constexpr int EPI = NC == 1 ? gu_epi_bytes<NT>() : 4 * QE_MFMA_MC * 4 + 16 * NT * (64 + 8 + 8);
+    static constexpr int ACT = DW + DW_SZ, ACT_SZ = 16 * NT * 128 > EPI ? 16 * NT * 128 : EPI;
     static constexpr int XS = ACT + 2 * ACT_SZ, XS_SZ = 4 * 16 * NT * 4;
     static constexpr int SIZE = XS + 2 * XS_SZ;
-    static_assert(EPI <= ACT_SZ, "the epilogue fits one stage");
 };
 struct ExpertSmem {
-    alignas(16) uint8_t raw[TileLds::SIZE];
+    static constexpr int SIZE = TileLds<2, 4>::SIZE;
+    static_assert(TileLds<1, 2>::SIZE <= SIZE, "the one-matrix waves fit as well");
+    alignas(16) uint8_t raw[SIZE];
     int pair[QE_MFMA_MC];
 };
 
-// Gate/up of a big item (33..64 pairs): wave = NC = 2 column groups of 16 weight rows
-// (gate, up) x NT = 4 16-pair tiles (NC MFMAs per block and tile; each weight decoded
-// once per item).  Workgroup yb (4 waves): h rows 16 (4 yb + wave) + 0..15; a 32-block
-// of h spans the wave pair (2w, 2w+1), which meets in LDS for its maximum.
+// Gate/up of an item, activations staged through LDS: wave = NC column groups of 16
+// weight rows x NT 16-pair tiles (NC MFMAs per block and tile; each weight decoded
+// once per item).  Row groups yb of a workgroup (4 waves):
+//   NC = 2 (33..64 pairs): h rows 16 (4 yb + wave) + 0..15; groups gate, up -- a
+//            32-block of h spans the wave pair (2w, 2w+1), which meets in LDS for its
+//            maximum;
+//   NC = 1 (fewer): h rows 32 yb + 16 (wave % 2) + 0..15 of the gate (waves 0, 1) or up
+//            (waves 2, 3) matrix -- half the rows of NC = 2 per workgroup, each
+//            output's K order unchanged.
+template <int NC, int NT>
 __device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it, const int yb, ExpertSmem &sm) {
-    constexpr int NC = 2, NT = TileLds::NT;
-    constexpr int KD = QE_D, NB = TileLds::NB; // reduction length, K blocks
+    static_assert(NC == 2 || NC == 1, "one or two column groups per wave");
+    constexpr int KD = QE_D, NB = QE_D / 32;   // reduction length, K blocks
     constexpr int NCH = NB / 8;                // turns (two quads each)
     constexpr uint32_t RB = QE_GU_ROW_BYTES;
     auto &s_pair = sm.pair;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, n = lane & 15, g = lane >> 4;
-    auto row_of = [&](int w, int c, int nn) -> int { return (c == 0 ? 0 : QE_FF_EXP) + (yb * 4 + w) * 16 + nn; };
+    auto row_of = [&](int w, int c, int nn) -> int {
+        if constexpr (NC == 2) return (c == 0 ? 0 : QE_FF_EXP) + (yb * 4 + w) * 16 + nn;
+        else return (w < 2 ? 0 : QE_FF_EXP) + (yb * 2 + (w & 1)) * 16 + nn;
+    };
     const uint8_t *ebase = a.arena + (size_t)it.x * QE_EXPERT_BYTES;
     // Buffer loads: a range-checked resource per operand (reads past the end
     // return 0), uniform per-turn offsets in SGPRs, per-lane offsets fixed.
@@ -165,7 +247,7 @@ __device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it
         const qe_u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, vo, so, 0);
         return make_uint4(v.x, v.y, v.z, v.w);
     };
-    using LY = TileLds;
+    using LY = TileLds<NC, NT>;
     uint8_t *const lds = sm.raw;
 
     uint32_t boff[NC]; // byte offset of block g of the lane's row, per column group
@@ -281,7 +363,10 @@ __device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it
             }
             {
                 uint32_t dep;
-                asm volatile("v_mov_b32 %0, 0" : "=v"(dep) : "v"(cw[0][0]), "v"(cw[1][0]));
+                if constexpr (NC == 2)
+                    asm volatile("v_mov_b32 %0, 0" : "=v"(dep) : "v"(cw[0][0]), "v"(cw[1][0]));
+                else
+                    asm volatile("v_mov_b32 %0, 0" : "=v"(dep) : "v"(cw[0][0]));
                 load_q(nx, qs, dep);
                 __builtin_amdgcn_sched_barrier(0);
             }
@@ -362,60 +447,65 @@ __device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it
     // the last quad (odd) read stage 1: the epilogue works in stage 0
 
     // lane holds rows 16 t + 4 g + i, column n of each group
-    // h rows 16 (4 yb + wv) + n: half (wv & 1) of 32-block jb
-    const int jb = yb * 2 + (wv >> 1), half = wv & 1;
-    // each wave's |h| maximum per pair, in the activation stage the last turn
-    // did not read (stage 0: its last reader passed the barrier that ended quad 2 NCH - 2)
-    float(*amax)[QE_MFMA_MC] = (float(*)[QE_MFMA_MC])(sm.raw + LY::ACT);
-    static_assert(4 * QE_MFMA_MC * 4 <= LY::ACT_SZ, "maxima fit one stage");
-    float h[NT][4], m[NT][4];
+    if constexpr (NC == 1) {
+        one_matrix_epilogue<NT>(a, yb, s_pair, acc[0], lds + LY::ACT); // stage 0, which the last quad did not read
+        return;
+    } else {
+        // h rows 16 (4 yb + wv) + n: half (wv & 1) of 32-block jb
+        const int jb = yb * 2 + (wv >> 1), half = wv & 1;
+        // each wave's |h| maximum per pair, in the activation stage the last turn
+        // did not read (stage 0: its last reader passed the barrier that ended quad 2 NCH - 2)
+        float(*amax)[QE_MFMA_MC] = (float(*)[QE_MFMA_MC])(sm.raw + LY::ACT);
+        static_assert(4 * QE_MFMA_MC * 4 <= LY::ACT_SZ, "maxima fit one stage");
+        float h[NT][4], m[NT][4];
 #pragma unroll
-    for (int t = 0; t < NT; ++t)
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            h[t][i] = silu_mul(acc[0][t][i], acc[1][t][i]);
-            m[t][i] = max16_abs(h[t][i]);
-            if (n == 0) amax[wv][16 * t + 4 * g + i] = m[t][i];
+            for (int i = 0; i < 4; ++i) {
+                h[t][i] = silu_mul(acc[0][t][i], acc[1][t][i]);
+                m[t][i] = max16_abs(h[t][i]);
+                if (n == 0) amax[wv][16 * t + 4 * g + i] = m[t][i];
+            }
+        __syncthreads();
+        // The workgroup's h of a pair is the 64 contiguous bytes [64 yb, 64 yb + 64) of its
+        // row in the operand layout (blocks 2 yb, 2 yb + 1), and its two block scales are
+        // adjacent: both are assembled in LDS (after the maxima, in the same free stage)
+        // and stored 16 bytes per thread, instead of one byte per lane and value.
+        uint8_t *htile = sm.raw + LY::ACT + 4 * QE_MFMA_MC * 4; // [16 NT][64]
+        float *stile = (float *)(htile + 16 * NT * 64);                                  // [16 NT][2]
+        float *itile = stile + 16 * NT * 2;                                              // [2][16 NT] inverses
+        static_assert(4 * QE_MFMA_MC * 4 + 16 * NT * (64 + 8 + 8) <= LY::ACT_SZ, "h tile fits the free stage");
+        if (tid < 2 * 16 * NT) { // block (jb % 2 = wave pair) scale and its inverse, once per pair
+            const int pr = tid / (16 * NT), mi = tid % (16 * NT);
+            float d;
+            itile[tid] = quant_scale_inv(fmaxf(amax[2 * pr][mi], amax[2 * pr + 1][mi]), d);
+            stile[mi * 2 + pr] = d;
         }
-    __syncthreads();
-    // The workgroup's h of a pair is the 64 contiguous bytes [64 yb, 64 yb + 64) of its
-    // row in the operand layout (blocks 2 yb, 2 yb + 1), and its two block scales are
-    // adjacent: both are assembled in LDS (after the maxima, in the same free stage)
-    // and stored 16 bytes per thread, instead of one byte per lane and value.
-    uint8_t *htile = sm.raw + LY::ACT + 4 * QE_MFMA_MC * 4; // [16 NT][64]
-    float *stile = (float *)(htile + 16 * NT * 64);                                  // [16 NT][2]
-    float *itile = stile + 16 * NT * 2;                                              // [2][16 NT] inverses
-    static_assert(4 * QE_MFMA_MC * 4 + 16 * NT * (64 + 8 + 8) <= LY::ACT_SZ, "h tile fits the free stage");
-    if (tid < 2 * 16 * NT) { // block (jb % 2 = wave pair) scale and its inverse, once per pair
-        const int pr = tid / (16 * NT), mi = tid % (16 * NT);
-        float d;
-        itile[tid] = quant_scale_inv(fmaxf(amax[2 * pr][mi], amax[2 * pr + 1][mi]), d);
-        stile[mi * 2 + pr] = d;
-    }
-    __syncthreads();
+        __syncthreads();
 #pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        const float4 id4 = *(const float4 *)(itile + (wv >> 1) * 16 * NT + 16 * t + 4 * g);
-        const float id[4] = {id4.x, id4.y, id4.z, id4.w};
+        for (int t = 0; t < NT; ++t) {
+            const float4 id4 = *(const float4 *)(itile + (wv >> 1) * 16 * NT + 16 * t + 4 * g);
+            const float id[4] = {id4.x, id4.y, id4.z, id4.w};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int mi = 16 * t + 4 * g + i;
-            htile[mi * 64 + (n >> 2) * 16 + (jb & 1) * 8 + (n & 3) + 4 * half] = (uint8_t)quant_one(h[t][i], id[i]);
+            for (int i = 0; i < 4; ++i) {
+                const int mi = 16 * t + 4 * g + i;
+                htile[mi * 64 + (n >> 2) * 16 + (jb & 1) * 8 + (n & 3) + 4 * half] = (uint8_t)quant_one(h[t][i], id[i]);
+            }
         }
-    }
-    __syncthreads();
-    {   // thread (pair tid / 4, 16-byte part tid % 4)
-        const int mi = tid >> 2, q = tid & 3;
-        const int p = mi < 16 * NT ? s_pair[mi] : -1;
-        if (p >= 0) {
-            int8_t *hp = a.hq + (size_t)p * QE_FF_EXP + (jb >> 1) * 64 + 16 * q;
-            float *sp = a.hs + (size_t)p * (QE_FF_EXP / 32) + 2 * (jb >> 1);
-            if (a.item_done) { // fused launch: written through for its down workgroups
-                st_sc1(hp, *(const uint4 *)(htile + mi * 64 + 16 * q));
-                if (q == 0) st_sc1(sp, *(const uint2 *)(stile + mi * 2));
-            } else {
-                *(uint4 *)hp = *(const uint4 *)(htile + mi * 64 + 16 * q);
-                if (q == 0) *(float2 *)sp = *(const float2 *)(stile + mi * 2);
+        __syncthreads();
+        {   // thread (pair tid / 4, 16-byte part tid % 4)
+            const int mi = tid >> 2, q = tid & 3;
+            const int p = mi < 16 * NT ? s_pair[mi] : -1;
+            if (p >= 0) {
+                int8_t *hp = a.hq + (size_t)p * QE_FF_EXP + (jb >> 1) * 64 + 16 * q;
+                float *sp = a.hs + (size_t)p * (QE_FF_EXP / 32) + 2 * (jb >> 1);
+                if (a.item_done) { // fused launch: written through for its down workgroups
+                    st_sc1(hp, *(const uint4 *)(htile + mi * 64 + 16 * q));
+                    if (q == 0) st_sc1(sp, *(const uint2 *)(stile + mi * 2));
+                } else {
+                    *(uint4 *)hp = *(const uint4 *)(htile + mi * 64 + 16 * q);
+                    if (q == 0) *(float2 *)sp = *(const float2 *)(stile + mi * 2);
+                }
             }
         }
     }
@@ -435,12 +525,12 @@ template <int NT> struct GuSmallLds {
     static constexpr int NB = QE_D / 32;
     static constexpr int DW = 0, XS = DW + NB * 64 * 2; // fp16 [block][wave][n]; fp32 [block][pair]
     static constexpr int EPI = XS + NB * 16 * NT * 4;
-    static constexpr int SIZE = EPI + (2 * 16 * 16 * 4 + 2 * 16 * 4 + 16 * 32 + 2 * 16 * 4) * NT;
+    static constexpr int SIZE = EPI + gu_epi_bytes<NT>();
 };
 template <int NT>
 __device__ __forceinline__ void gu_small(const GemmTileArgs &a, const int4 it, const int yb, ExpertSmem &sm) {
     using LY = GuSmallLds<NT>;
-    static_assert(LY::SIZE <= TileLds::SIZE, "the small items' tile fits as well");
+    static_assert(LY::SIZE <= ExpertSmem::SIZE, "the small items' tile fits as well");
     constexpr int NB = LY::NB, NQ = NB / 4, RC = 4, RA = 4 / NT;
     constexpr uint32_t RB = QE_GU_ROW_BYTES;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, n = lane & 15, g = lane >> 4;
@@ -557,75 +647,14 @@ __device__ __forceinline__ void gu_small(const GemmTileArgs &a, const int4 it, c
 #pragma unroll
     for (int s = 0; s < RC; ++s) quad(NQ - RC + s, s, s % RA, false, s + RA < RC);
 
-    // 32-block yb of h: rows 16 rs + n, rs = wv % 2, from gate wave rs and up wave
-    // 2 + rs
-    uint8_t *fs = lds + LY::EPI;
-    float *utile = (float *)fs;                              // [2][16 NT pairs][16] the up dots
-    float *amax = utile + 2 * 16 * NT * 16;                  // [2][16 NT] |h| maxima per half
-    uint8_t *htile = (uint8_t *)(amax + 2 * 16 * NT);         // [16 NT][32] int8 h, operand order
-    float *stile = (float *)(htile + 16 * NT * 32);          // [16 NT] block scales
-    float *itile = stile + 16 * NT;                          // [16 NT] their inverses
-    const int rs = wv & 1;
-    if (wv >= 2) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) utile[(rs * 16 * NT + 16 * t + 4 * g + i) * 16 + n] = acc[t][i];
-    }
-    __syncthreads();
-    float h[NT][4], m[NT][4];
-    if (wv < 2) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int mi = 16 * t + 4 * g + i;
-                h[t][i] = silu_mul(acc[t][i], utile[(rs * 16 * NT + mi) * 16 + n]);
-                m[t][i] = max16_abs(h[t][i]);
-                if (n == 0) amax[rs * 16 * NT + mi] = m[t][i];
-            }
-    }
-    __syncthreads();
-    if (tid < 16 * NT) { // the block's scale and its inverse, once per pair
-        float d;
-        itile[tid] = quant_scale_inv(fmaxf(amax[tid], amax[16 * NT + tid]), d);
-        stile[tid] = d;
-    }
-    __syncthreads();
-    if (wv < 2) {
-        // element 16 rs + n of the block: byte (n / 4) * 16 + (yb % 2) * 8 + n % 4 + 4 rs
-        // of the pair's 64-byte run (yb / 2) of h (as expert_tile);
-        // htile keeps this block's 8-byte groups n / 4 contiguous
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int mi = 16 * t + 4 * g + i;
-                htile[mi * 32 + (n >> 2) * 8 + (n & 3) + 4 * rs] = (uint8_t)quant_one(h[t][i], itile[mi]);
-            }
-    }
-    __syncthreads();
-    {   // thread (pair tid / 4, 8-byte group tid % 4)
-        const int mi = tid >> 2, q = tid & 3;
-        const int p = mi < 16 * NT ? s_pair[mi] : -1;
-        if (p >= 0) {
-            int8_t *hp = a.hq + (size_t)p * QE_FF_EXP + (yb >> 1) * 64 + 16 * q + 8 * (yb & 1);
-            float *sp = a.hs + (size_t)p * (QE_FF_EXP / 32) + yb;
-            if (a.item_done) { // fused launch: written through for its down workgroups
-                st_sc1(hp, *(const uint2 *)(htile + mi * 32 + 8 * q));
-                if (q == 0) st_sc1(sp, stile[mi]);
-            } else {
-                *(uint2 *)hp = *(const uint2 *)(htile + mi * 32 + 8 * q);
-                if (q == 0) *sp = stile[mi];
-            }
-        }
-    }
+    one_matrix_epilogue<NT>(a, yb, s_pair, acc, lds + LY::EPI);
 }
 
 // Gate/up: big items (33..64 pairs, the first n_items[1]) run NT = 4, NC = 2
-// on 8 row groups of 64 h rows; the small ones after them gu_small on
-// 16 row groups of 32 h rows: twice the workgroups of half the life (these items
-// run last, after the big ones, and their workgroups had made the launch's tail).  Workgroup b runs on XCD x = b % 8 (round-robin dispatch) and
+// on 8 row groups of 64 h rows; the small ones after them (NC = 1, or gu_small in
+// small calls) on 16 row groups of 32 h rows: twice the workgroups of half the life
+// (these items run last, after the big ones, and their workgroups had made the
+// launch's tail).  Workgroup b runs on XCD x = b % 8 (round-robin dispatch) and
 // takes the (b / 8)-th row group of that XCD's items x, x + 8, ..., the big
 // ones' first: all row groups of an item run on one XCD, so its activations
 // come from HBM once and from that XCD's L2 after.  (The odd row groups of a
@@ -642,11 +671,11 @@ QE_DEV void expert_unit(const GemmTileArgs &a, int b, ExpertSmem &sm) {
     const int4 it = a.items[item];
     static_assert(QE_MFMA_MC == 64, "items of up to four 16-row tiles");
     if (big)
-        expert_tile(a, it, yb, sm);
-    else if (it.z > 16)
-        gu_small<2>(a, it, yb, sm);
+        expert_tile<2, 4>(a, it, yb, sm);
+    else if (a.direct)
+        it.z > 16 ? gu_small<2>(a, it, yb, sm) : gu_small<1>(a, it, yb, sm);
     else
-        gu_small<1>(a, it, yb, sm);
+        it.z > 16 ? expert_tile<1, 2>(a, it, yb, sm) : expert_tile<1, 1>(a, it, yb, sm);
     if (a.item_done) {
         // fused launch: every thread's h stores (sc1, written through) are acknowledged
         // before the item's count of finished gate/up workgroups goes up
@@ -1500,6 +1529,11 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
     GemmTileArgs g{};
     g.arena = L.arena; g.pairs = S.pairs; g.items = S.items; g.n_items = S.n_items; g.wts = S.wts;
     g.aq = S.xqp; g.a_bytes = T * QE_D; g.as = S.xs; g.a_row_div = QE_K_USED; g.hq = S.hqp; g.hs = S.hs;
+    // Below 256 tokens most items hold a few pairs and their weights' latency decides:
+    // activations straight to registers (100 tokens 157 -> 149 us).  With more pairs the
+    // four waves' separate reads of them cost more than the staging (1000 tokens 241 us
+    // staged, 260 direct).
+    g.direct = T < 256;
     const bool fused = T >= QE_FUSE_T_MIN && T < QE_FUSE_T && S.item_done;
     if (fused) {
         g.item_done = S.item_done; g.err = S.err; g.err_val = S.err_val; g.spin_cap = S.spin_cap;
