@@ -722,6 +722,19 @@ __global__ __launch_bounds__(256, 4) void k_expert_gu(GemmTileArgs a) {
 typedef float qe_float16v __attribute__((ext_vector_type(16)));
 #define SH_GU_KB 8 /* 32-blocks per wave in gate/up: 2048 / 32 / 8 */
 
+// Shared-expert tiles over the XCDs: mt token tiles x nt row tiles (a multiple of 8).
+// With 5 token tiles or more, a token tile's row tiles run on one XCD back to back
+// (its activations reach one L2); with fewer, that would leave half the XCDs or more
+// without any, and the row tiles are dealt over all eight, each reading its share of
+// the weights (k_router_shgu at 12 tokens 14.2 -> 8.8 us, at 100 tokens 14.4 -> 9.9;
+// at 200 tokens, 7 token tiles, the first form is the faster by 1 us).
+QE_HD int xcd_tiles(int mt, int nt, int x) { return mt < 5 ? mt * nt / 8 : nt * ((mt - x + 7) / 8); }
+QE_DEV void xcd_tile(int mt, int nt, int x, int k, int &m, int &n) { // the k-th tile of XCD x
+    const int s = 8 * k + x;
+    m = mt < 5 ? s / nt : 8 * (k / nt) + x;
+    n = mt < 5 ? s % nt : k % nt;
+}
+
 QE_DEV qe_u32x4 sh_ld(__amdgpu_buffer_rsrc_t r, uint32_t off) { return __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, 0); }
 
 // one 32-block: acc += dw * (A_hi + A_lo) . B, A = a[0..3] (hi 0..7, hi 8..15, lo 0..7, lo 8..15)
@@ -950,7 +963,7 @@ QE_DEV void shgu_tile(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *hh
 // tile, K split) and the 32 shared gate/up row tiles of one token tile.
 constexpr int RS_JT = QE_FF_SH / 16;
 QE_HD int rs_router_per_xcd(int T, int nz, int x) { return 2 * (((T + 63) / 64 * nz - x + 7) / 8); }
-QE_HD int rs_shgu_per_xcd(int T, int x) { return RS_JT * (((T + 31) / 32 - x + 7) / 8); }
+QE_HD int rs_shgu_per_xcd(int T, int x) { return xcd_tiles((T + 31) / 32, RS_JT, x); }
 template <int LEV>
 __global__ __launch_bounds__(512, 4) void k_router_shgu(const float *xn, const _Float16 *xhl, int T, const float *Wr,
                                                         const uint8_t *Wg, float *part, _Float16 *hhl) {
@@ -976,7 +989,9 @@ __global__ __launch_bounds__(512, 4) void k_router_shgu(const float *xn, const _
         router_tile<LEV, 4, 1>(xn, T, Wr, part, g / NZ, idx & 1, g % NZ, sm.r);
     } else {
         if (idx >= ns) return;
-        shgu_tile(xhl, T, Wg, hhl, 8 * (idx / RS_JT) + x, idx % RS_JT, sm.s);
+        int m, j;
+        xcd_tile((T + 31) / 32, RS_JT, x, idx, m, j);
+        shgu_tile(xhl, T, Wg, hhl, m, j, sm.s);
     }
 }
 
@@ -1428,25 +1443,25 @@ __device__ __forceinline__ void dn_unit(const GemmTileArgs &a, int b, DnSmem &sm
 // workgroups of the routed down over the items of np pairs (as expert_max_wg)
 QE_HD int dn_max_wg(int np, int rgw) { return ((QE_D / 128) / rgw) * (((np / (QE_MFMA_MC / 2 + 1) + 1 + QE_N_EXPERT) + 7) & ~7); }
 
-// Routed down items and shared down tiles in one launch: the routed items
-// (item, then row-group block) come first, the shared tiles fill the CUs as the
-// routed work drains.
-__global__ __launch_bounds__(256, 2) void k_expert_dn(GemmTileArgs a, int nr, const _Float16 *hhl, int T,
+// Routed down items and shared down tiles in one launch.  At large T the routed
+// items (item, then row-group block) come first and the shared tiles fill the CUs as
+// the routed work drains (sh0 = nr); below QE_FUSE_T_MIN tokens there are few
+// shared tiles, each a longer chain than a routed workgroup, and they come first
+// (sh0 = 0; last, they ran alone at the end: 28.3 us against 20.2 at 12 tokens).
+__global__ __launch_bounds__(256, 2) void k_expert_dn(GemmTileArgs a, int nr, int sh0, int nsh, const _Float16 *hhl, int T,
                                                       const uint8_t *Wsd, float *sd) {
     __shared__ union {
         DnSmem d;
         Shdn64Lds s;
     } sm;
-    const int b = blockIdx.x;
-    if (b < nr) {
-        dn_unit(a, b, sm.d);
+    const int b = blockIdx.x, s = b - sh0; // nr and nsh are multiples of 8: b % 8 is the XCD of either kind
+    if (s < 0 || s >= nsh) {
+        dn_unit(a, s < 0 ? b : b - nsh, sm.d);
     } else {
-        const int s = b - nr;
-        // tile s runs on XCD s % 8 (nr is a multiple of 8 below): the 16 column
-        // tiles of one 64-token pair back to back there
-        const int x = s & 7, k = s >> 3, mp = 8 * (k / (QE_D / 128)) + x;
+        int mp, n;
+        xcd_tile((T + 63) / 64, QE_D / 128, s & 7, s >> 3, mp, n);
         if (mp >= (T + 63) / 64) return;
-        shdn_tile64(hhl, T, Wsd, sd, mp, k % (QE_D / 128), (uint8_t *)&sm.s);
+        shdn_tile64(hhl, T, Wsd, sd, mp, n, (uint8_t *)&sm.s);
     }
 }
 
@@ -1483,10 +1498,11 @@ __global__ __launch_bounds__(256, 4) void k_expert_gudn(GemmTileArgs gu, GemmTil
         return;
     }
     int r = k - gux;
-    if (r < nshx) { // shared tile s = 8 r + x: the 16 column tiles of one 64-token pair back to back
-        const int mp = 8 * (r / (QE_D / 128)) + x;
+    if (r < nshx) { // the XCD's shared tiles
+        int mp, n;
+        xcd_tile((T + 63) / 64, QE_D / 128, x, r, mp, n);
         if (mp >= (T + 63) / 64) return;
-        shdn_tile64(hhl, T, Wsd, sd, mp, r % (QE_D / 128), (uint8_t *)&sm.s);
+        shdn_tile64(hhl, T, Wsd, sd, mp, n, (uint8_t *)&sm.s);
         return;
     }
     r -= nshx;
@@ -1548,7 +1564,7 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
     // (4 from 256 tokens in separate launches: measured best at 512 and 8192; fused,
     // shorter down workgroups drain the tail sooner: 1 below 512 tokens, then 2)
     d.dn_rgw = fused ? (T < 512 ? 1 : 2) : T >= QE_DN_RGW4_T ? 4 : T >= QE_DN_RGW2_T ? 2 : 1;
-    const int nsh = 8 * (QE_D / 128) * (((T + 63) / 64 + 7) / 8);
+    const int nsh = 8 * xcd_tiles((T + 63) / 64, QE_D / 128, 0);
     const int nr = dn_max_wg(np, d.dn_rgw); // a multiple of 8: shared tiles start on XCD 0
     if (fused) {
         // per XCD at most: 16 gate/up and rgb_n down workgroups for each of its items, and its shared tiles
@@ -1556,6 +1572,6 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
         k_expert_gudn<<<8 * ((16 + rgb_n) * ix + nsh / 8), 256, 0, st>>>(g, d, nsh / 8, (const _Float16 *)S.shgu, T,
                                                                           L.sh_dn, S.sd);
     } else
-        k_expert_dn<<<nr + nsh, 256, 0, st>>>(d, nr, (const _Float16 *)S.shgu, T, L.sh_dn, S.sd);
+        k_expert_dn<<<nr + nsh, 256, 0, st>>>(d, nr, T < QE_FUSE_T_MIN ? 0 : nr, nsh, (const _Float16 *)S.shgu, T, L.sh_dn, S.sd);
     return hipGetLastError();
 }
