@@ -25,6 +25,16 @@ static inline size_t qe_rpart_rows(size_t t_max) { // token rows of partials tha
 }
 #define QE_MFMA_MC 64 /* pairs per work item of the prefill MFMA grouped GEMMs (up to four 16-row tiles) */
 
+// Pairs per work item at T tokens.  Small calls fill the GPU with few workgroups, and
+// an expert's 33..64 pairs in one item made the longest of them (36 us alone, 50 in
+// company): items of 32 halve that (us per layer, skewed routing: 100 tokens 105 -> 88,
+// 200 tokens 113 -> 98).  With more tokens the second decode of the weights costs more
+// (250 tokens 106.6 -> 107.4, 400 tokens 155 -> 185).
+#define QE_ITEM32_T 224
+static inline int qe_item_pairs(int T) { return T < QE_ITEM32_T ? 32 : QE_MFMA_MC; }
+// upper bound of the items of T tokens: those of more than half the pairs, and one
+// smaller per expert
+static inline int qe_max_items(int T) { return T * QE_K_USED / (qe_item_pairs(T) / 2 + 1) + 1 + QE_N_EXPERT; }
 
 // One layer's weights inside the context.
 struct QeLayerPtrs {
@@ -73,7 +83,7 @@ struct QeScratch {
     float *rpart;                           // [nz][T][256] router subtree partials (qe_router_splits)
     int32_t *ids; float *wts; float *shg;   // [T][8], [T][8], [T]
     int32_t *off; int32_t *pairs;           // [257], [T*8]
-    int4 *items; int32_t *n_items;          // work items (expert, first pair, count); n_items[0] items, the first n_items[1] big
+    int4 *items; int32_t *n_items;          // work items (expert, first pair, count); n_items[0] items, the first n_items[1] of more than 32 pairs
     int8_t *hqp; float *hs;                 // [T*8][512] quantised h (operand layout), [T*8][16] scales
     float *sd;                              // [T][2048] shared-expert output
     float *yp;                              // [T*8][2048] weighted expert outputs

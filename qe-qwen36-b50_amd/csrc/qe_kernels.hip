@@ -174,9 +174,9 @@ __global__ __launch_bounds__(1024) void k_disp_hist(const int32_t *ids, int np, 
 // Dispatch pass 2: offsets and the stable scatter (engine/qe.cpp:1968-1976).
 // Inside a chunk, a pair's rank among earlier same-expert pairs is the count
 // in earlier waves plus its rank in its own wave (8 ballots on the id bits).
-// Block 0 also writes off[] and the work items (expert, first pair, count <= TC):
-// those of more than TC / 2 pairs first, n_items[0] items in all, n_items[1] of
-// them big.
+// Block 0 also writes off[] and the work items (expert, first pair, count <= TC, 64 or
+// 32): those of more than TC / 2 pairs first, n_items[0] items in all, n_items[1] of
+// them of more than 32 pairs.
 __global__ __launch_bounds__(1024) void k_disp_scatter(const int32_t *ids, int np, const int32_t *chunk_hist, int nch,
                                                        int tc, int32_t *off_out, int32_t *pairs, int4 *items,
                                                        int32_t *n_items, int32_t *item_done) {
@@ -261,7 +261,7 @@ __global__ __launch_bounds__(1024) void k_disp_scatter(const int32_t *ids, int n
         if (ns) items[all_b + is - 1] = make_int4(tid, off + full * tc, rem, 0);
         if (tid == QE_N_EXPERT - 1) {
             n_items[0] = all_b + all_s;
-            n_items[1] = all_b;
+            n_items[1] = tc == QE_MFMA_MC ? all_b : 0; // of more than 32 pairs
         }
         if (item_done) // the fused gate/up + down launch counts its gate/up workgroups per item
             for (int i = tid; i < all_b + all_s; i += QE_N_EXPERT) item_done[i] = 0;
@@ -425,7 +425,7 @@ hipError_t qe_launch_layer(const QeLayerPtrs &L, const QeScratch &S, const float
     {
         QE_PROF(QP_DISPATCH); // the histogram came with k_topk
         const int np = T * QE_K_USED, nch = (np + 1023) / 1024;
-        k_disp_scatter<<<nch, 1024, 0, st>>>(S.ids, np, S.chunk_hist, nch, QE_MFMA_MC, S.off, S.pairs, S.items,
+        k_disp_scatter<<<nch, 1024, 0, st>>>(S.ids, np, S.chunk_hist, nch, qe_item_pairs(T), S.off, S.pairs, S.items,
                                               S.n_items, S.item_done);
     }
     {

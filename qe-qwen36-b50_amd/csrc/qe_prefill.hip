@@ -684,12 +684,9 @@ QE_DEV void expert_unit(const GemmTileArgs &a, int b, ExpertSmem &sm) {
         if (threadIdx.x == 0) __hip_atomic_fetch_add(a.item_done + item, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
 }
-// Workgroups over the items of np pairs: an upper bound of the item count
-// (items of more than QE_MFMA_MC / 2 pairs, plus at most one smaller item per
-// expert) rounded up to whole groups of 8 items, times the row groups.
-constexpr int expert_max_wg(int np) {
-    return QE_FF_EXP / 32 * (((np / (QE_MFMA_MC / 2 + 1) + 1 + QE_N_EXPERT) + 7) & ~7);
-}
+// Workgroups over the items of T tokens: their upper bound rounded up to whole groups
+// of 8 items, times the row groups.
+static int expert_max_wg(int T) { return QE_FF_EXP / 32 * ((qe_max_items(T) + 7) & ~7); }
 __global__ __launch_bounds__(256, 4) void k_expert_gu(GemmTileArgs a) {
     __shared__ ExpertSmem sm;
     expert_unit(a, blockIdx.x, sm);
@@ -1440,8 +1437,8 @@ __device__ __forceinline__ void dn_unit(const GemmTileArgs &a, int b, DnSmem &sm
     if (item >= a.n_items[0]) return;
     dn_unit_at<false>(a, item, rgb, sm);
 }
-// workgroups of the routed down over the items of np pairs (as expert_max_wg)
-QE_HD int dn_max_wg(int np, int rgw) { return ((QE_D / 128) / rgw) * (((np / (QE_MFMA_MC / 2 + 1) + 1 + QE_N_EXPERT) + 7) & ~7); }
+// workgroups of the routed down over the items of T tokens (as expert_max_wg)
+static int dn_max_wg(int T, int rgw) { return ((QE_D / 128) / rgw) * ((qe_max_items(T) + 7) & ~7); }
 
 // Routed down items and shared down tiles in one launch.  At large T the routed
 // items (item, then row-group block) come first and the shared tiles fill the CUs as
@@ -1555,7 +1552,7 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
         g.item_done = S.item_done; g.err = S.err; g.err_val = S.err_val; g.spin_cap = S.spin_cap;
         g.wait_extra = S.wait_extra;
     } else {
-        k_expert_gu<<<expert_max_wg(np), 256, 0, st>>>(g);
+        k_expert_gu<<<expert_max_wg(T), 256, 0, st>>>(g);
     }
     GemmTileArgs d = g;
     d.aq = S.hqp; d.a_bytes = np * QE_FF_EXP; d.as = S.hs; d.a_row_div = 1; d.yp = S.yp;
@@ -1565,10 +1562,10 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
     // shorter down workgroups drain the tail sooner: 1 below 512 tokens, then 2)
     d.dn_rgw = fused ? (T < 512 ? 1 : 2) : T >= QE_DN_RGW4_T ? 4 : T >= QE_DN_RGW2_T ? 2 : 1;
     const int nsh = 8 * xcd_tiles((T + 63) / 64, QE_D / 128, 0);
-    const int nr = dn_max_wg(np, d.dn_rgw); // a multiple of 8: shared tiles start on XCD 0
+    const int nr = dn_max_wg(T, d.dn_rgw); // a multiple of 8: shared tiles start on XCD 0
     if (fused) {
         // per XCD at most: 16 gate/up and rgb_n down workgroups for each of its items, and its shared tiles
-        const int ix = ((np / (QE_MFMA_MC / 2 + 1) + 1 + QE_N_EXPERT) + 7) / 8, rgb_n = (QE_D / 128) / d.dn_rgw;
+        const int ix = (qe_max_items(T) + 7) / 8, rgb_n = (QE_D / 128) / d.dn_rgw;
         k_expert_gudn<<<8 * ((16 + rgb_n) * ix + nsh / 8), 256, 0, st>>>(g, d, nsh / 8, (const _Float16 *)S.shgu, T,
                                                                           L.sh_dn, S.sd);
     } else
