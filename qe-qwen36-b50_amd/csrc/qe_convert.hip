@@ -14,11 +14,30 @@
 //   S_xq^2 > best*S_qq; the scale is stored as fp16 and the codes are the
 //   nearest entries of (1/d)*x_j with the fp32 d.
 //
-// Here one thread quantizes one block, with the fp32 operations of that
-// sequence in the same order (the library builds with -ffp-contract=off and
-// correctly rounded division), so the bytes are identical to the CPU
-// checker's.  The work is VALU-bound: 16 candidates x 32 elements against
-// 1.6 bytes of HBM traffic per element.
+// Here one thread quantizes one block, and the bytes are identical to the CPU
+// checker's (the library builds with -ffp-contract=off and correctly rounded
+// division).  Scoring all sixteen candidates with that sequence is 16 x 32 table reads
+// and about 5,000 VALU instructions per block; instead:
+//   * Over the fifteen scales s = -n/m, n = 120..134, an element's nearest entry changes
+//     at most once: neighbouring midpoints are more than a factor 134/120 apart (the
+//     closest, 115.5 and 93.5, a factor 1.235).  So two reads, at n = 120 and n = 134,
+//     give both entries; their sum, twice the midpoint between them, gives the n where
+//     the change happens, and one exact evaluation at the nearest integer decides
+//     between it and the next (every other n is further from the midpoint than rounding
+//     reaches).  Each change is added to the bin of its n; prefix sums over the bins give
+//     S_xq and S_qq of every candidate.  All their terms have one sign (bar an opposite
+//     entry 1, below 1e-4 of the sum), so the relative errors are at most the roundings
+//     on a term's way, of 2^-24 each: 2 + 31 in the sequence, 2 + 8 + 2 + 14 here, and up
+//     to 31 more on what met in one bin (at most 0.21 of S_xq and 0.35 of S_qq).
+//   * A candidate whose approximate score S_xq^2 / S_qq is below the largest by more than
+//     3e-5 (2 x 99 roundings of the sequence's score, 2 x 102 of this one: 2.4e-5, and the
+//     last operations) cannot be the last to win; what is left -- mostly one candidate --
+//     is evaluated with the fp32 operations of the sequence, in its order, starting from
+//     s0's exact score.  The first is evaluated by the block's own lane, the others by the
+//     wave's lanes in turn.  Candidates with no change between them assign alike and
+//     score alike, and only the first is evaluated.
+//   * Blocks whose largest element lies outside [1e-6, 1e4], where the products could
+//     underflow or overflow, or that hold a NaN, take the sequence over all sixteen.
 //
 // nearest(a): ggml bisects the codebook and keeps the lower of the two
 // bracketing entries when a - lo < hi - a.  Both differences are exact
@@ -74,13 +93,12 @@ template <typename T> __device__ inline T tab_at(const T *tab0, int bytes) {
 }
 
 // S_xq and S_qq of inverse scale s (given as s8 = 8 s), in element order
-__device__ inline void nl4_fit(const float (&x)[32], const float (&w)[32], float s8, const float *tab0, float &sxq,
-                               float &sqq) {
+__device__ inline void nl4_fit(const float (&x)[32], float s8, const float *tab0, float &sxq, float &sqq) {
     float a = 0.f, b = 0.f;
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
         const float q = tab_at(tab0, slot_bytes(s8 * x[j]));
-        const float wq = w[j] * q;
+        const float wq = (x[j] * x[j]) * q;
         a = a + wq * x[j];
         b = b + wq * q;
     }
@@ -126,39 +144,163 @@ __device__ inline void load_block(const uint8_t *src, uint32_t g, float (&x)[32]
     }
 }
 
-template <int TYPE>
-__global__ __launch_bounds__(256) void k_nl4_quant(QeNl4Args a) {
+// 8 n / -m for n = 120..134, correctly rounded, from mn = -m / 8 and rn = 1 / mn: the
+// quotient estimate and one remainder step (equal to the division for all 2^23
+// mantissas of m and every n, checked exhaustively; no exponent in use here over- or
+// underflows).
+__device__ inline float scale8(float n, float mn, float rn) {
+    const float q = n * rn;
+    return fmaf(fmaf(-q, mn, n), rn, q);
+}
+
+// WPS: waves per SIMD the registers are cut for (qe_launch_nl4_quant).
+// What bounds it: VALU issue (3,075 instructions a block of 64 threads, of half rate
+// where they convert, clamp or mask) and the slot reads' bank conflicts (a third of the
+// cycles).  One Q8_0 layer (25 M blocks): 2,440 us scoring all candidates, 1,590 now;
+// 16,384 bf16 blocks 14.8 -> 11.5 us.  Measured on the way: the bins by LDS float atomics
+// 9,020 us; every lane evaluating its own remaining candidates 1,750 (four rounds a wave
+// instead of about 1.4).
+template <int TYPE, int WPS>
+__global__ __launch_bounds__(256, WPS) void k_nl4_quant(QeNl4Args a) {
+    constexpr int N0 = 120, NC = 15; // candidates s = -n/m, n = N0 .. N0 + NC - 1 (t = 127 - n)
     __shared__ float s_q[NL4_SLOTS];
     __shared__ int s_c[NL4_SLOTS];
+    __shared__ float2 s_bin[NC - 1][256]; // [n - N0 - 1][thread]: what S_xq, S_qq change by from n - 1 to n
     build_table(s_q, s_c);
     __syncthreads();
     const uint32_t g = blockIdx.x * 256u + threadIdx.x;
-    if (g >= a.nblk) return;
-    float x[32], w[32];
-    load_block<TYPE>(a.src, g, x);
+    const bool live = g < a.nblk; // lanes past the end stay for the wave's exchange
+    float x[32];
+    if (live) {
+        load_block<TYPE>(a.src, g, x);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 32; ++j) x[j] = 0.f;
+    }
     const float *q0 = s_q + NL4_HALF;
 
     float amax = 0.f, m = 0.f;
 #pragma unroll
     for (int j = 0; j < 32; ++j) {
-        w[j] = x[j] * x[j];
         if (fabsf(x[j]) > amax) { amax = fabsf(x[j]); m = x[j]; }
     }
-    float d = 0.f;
+    float d = 0.f, best_rest = 0.f;
+    uint32_t rest = 0u; // candidates left after the first
     if (amax >= 1e-15f) {
         float sxq, sqq;
-        nl4_fit(x, w, 8.f * (1.f / (m / 127.f)), q0, sxq, sqq);
+        nl4_fit(x, 8.f * (1.f / (m / 127.f)), q0, sxq, sqq);
         d = sxq / sqq;
         float best = d * sxq;
-#pragma unroll 1
-        for (int t = -7; t <= 7; ++t) {
-            nl4_fit(x, w, 8.f * ((float)(t - 127) / m), q0, sxq, sqq);
+        uint32_t cand = (1u << NC) - 1u; // candidates to evaluate, bit n - N0
+        const float mn = -0.125f * m, rn = 1.f / mn;
+        if (amax >= 1e-6f && amax <= 1e4f) {
+            float2 *bin = &s_bin[0][threadIdx.x]; // this thread's column
+#pragma unroll
+            for (int i = 0; i < NC - 1; ++i) bin[256 * i] = make_float2(0.f, 0.f);
+            const float slo = scale8((float)N0, mn, rn), shi = scale8((float)(N0 + NC - 1), mn, rn), hm = 4.f * mn;
+            float A4[4] = {0.f, 0.f, 0.f, 0.f}, B4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < 32; ++j) {
+                const float ql = tab_at(q0, slot_bytes(slo * x[j])), qh = tab_at(q0, slot_bytes(shi * x[j]));
+                const float sum = ql + qh, dq = qh - ql;
+                const float w = x[j] * x[j], p = w * x[j];
+                A4[j & 3] = fmaf(p, ql, A4[j & 3]);
+                B4[j & 3] = fmaf(w * ql, ql, B4[j & 3]);
+                // the change lies at n = (ql + qh) / 2 * -m / x; without one (or x = 0) the
+                // result is any bin and nothing is added
+                const float n0 = rintf(fminf(fmaxf(sum * hm * __builtin_amdgcn_rcpf(x[j]), (float)N0), (float)(N0 + NC - 1)));
+                const bool outer = (scale8(n0, mn, rn) * x[j] >= 4.f * sum) == (dq > 0.f); // at n0 already qh
+                const int i = min((int)n0 - N0 - 1 + (outer ? 0 : 1), NC - 2);
+                float2 *bj = bin + 256 * max(i, 0);
+                const float2 v = *bj;
+                *bj = make_float2(fmaf(p, dq, v.x), fmaf(w * dq, sum, v.y));
+            }
+            float A = (A4[0] + A4[1]) + (A4[2] + A4[3]), B = (B4[0] + B4[1]) + (B4[2] + B4[3]);
+            float sc[NC], top = sxq * sxq * __builtin_amdgcn_rcpf(sqq);
+            uint32_t same = 0u; // bit n - N0: n assigns as n + 1 does
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                if (i > 0) {
+                    const float2 v = bin[256 * (i - 1)];
+                    if (A + v.x == A) same |= 1u << (i - 1);
+                    A += v.x;
+                    B += v.y;
+                }
+                sc[i] = A * A * __builtin_amdgcn_rcpf(B);
+                top = fmaxf(top, sc[i]);
+            }
+            if (A == A) { // no NaN in the block
+                const float thr = top * (1.f - 3e-5f);
+                cand = 0u;
+#pragma unroll
+                for (int i = 0; i < NC; ++i)
+                    if (sc[i] >= thr) cand |= 1u << i;
+                cand &= ~same;
+            }
+        }
+        // in the sequence's order, n from 134 down (the general division: this also serves
+        // blocks outside scale8's range); the first one here, the others -- about one
+        // block in three has any -- dealt over the lanes of the wave
+        if (cand) {
+            const int i = 31 - __builtin_clz(cand);
+            cand &= ~(1u << i);
+            nl4_fit(x, 8.f * ((float)(-N0 - i) / m), q0, sxq, sqq);
             if (sqq > 0.f && sxq * sxq > best * sqq) {
                 d = sxq / sqq;
                 best = d * sxq;
             }
         }
+        rest = cand;
+        best_rest = best;
     }
+    {
+        // The wave's list of (lane, candidate), in its lanes' bins (64 columns of 14
+        // slots, read out by now): an entry is evaluated by lane k % 64, from the block in
+        // memory, and replaced by its sums, which the owner takes in order.
+        const int lane = threadIdx.x & 63, cnt = __popc(rest);
+        int off = cnt;
+#pragma unroll
+        for (int s = 1; s < 64; s <<= 1) {
+            const int v = __shfl_up(off, s);
+            if (lane >= s) off += v;
+        }
+        const int total = __builtin_amdgcn_readlane(off, 63);
+        off -= cnt;
+        float2 *wbin = &s_bin[0][threadIdx.x & ~63]; // slot k: row k / 64, column k % 64 of the wave
+        auto slot = [&](int k) -> float2 & { return wbin[256 * (k >> 6) + (k & 63)]; };
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        uint32_t left = rest;
+        for (int k = off; left; ++k) {
+            const int i = 31 - __builtin_clz(left);
+            left &= ~(1u << i);
+            slot(k) = make_float2(__int_as_float(lane), __int_as_float(i));
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int k0 = 0; k0 < total; k0 += 64) {
+            const int k = k0 + lane;
+            const float2 e = k < total ? slot(k) : make_float2(__int_as_float(lane), 0.f);
+            const int o = __float_as_int(e.x) & 63;
+            const float mo = __shfl(m, o);
+            if (k < total) {
+                float y[32], sxq, sqq;
+                load_block<TYPE>(a.src, g - lane + o, y);
+                nl4_fit(y, 8.f * ((float)(-N0 - __float_as_int(e.y)) / mo), q0, sxq, sqq);
+                slot(k) = make_float2(sxq, sqq);
+            }
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        for (int k = off; k < off + cnt; ++k) {
+            const float2 v = slot(k);
+            if (v.y > 0.f && v.x * v.x > best_rest * v.y) {
+                d = v.x / v.y;
+                best_rest = d * v.x;
+            }
+        }
+    }
+    if (!live) return;
     const float s8 = 8.f * (d != 0.f ? 1.f / d : 0.f);
     const int *c0 = s_c + NL4_HALF;
     uint32_t c[4] = {0u, 0u, 0u, 0u};
@@ -180,11 +322,18 @@ __global__ __launch_bounds__(256) void k_nl4_quant(QeNl4Args a) {
 hipError_t qe_launch_nl4_quant(const QeNl4Args &a, int src_type, hipStream_t st) {
     if (a.nblk == 0) return hipSuccess;
     const dim3 grid((a.nblk + 255) / 256), block(256);
+    // up to three workgroups per CU: all run at once, and what counts is one wave's own
+    // pace, which more registers help (16,384 blocks 13.0 -> 11.5 us); beyond, the fourth
+    // wave per SIMD does (25 M blocks 1,727 -> 1,590)
+    const auto go = [&](auto small, auto large) {
+        if (grid.x <= 3 * 256) small<<<grid, block, 0, st>>>(a);
+        else large<<<grid, block, 0, st>>>(a);
+    };
     switch (src_type) {
-    case QE_SRC_F32: k_nl4_quant<QE_SRC_F32><<<grid, block, 0, st>>>(a); break;
-    case QE_SRC_F16: k_nl4_quant<QE_SRC_F16><<<grid, block, 0, st>>>(a); break;
-    case QE_SRC_BF16: k_nl4_quant<QE_SRC_BF16><<<grid, block, 0, st>>>(a); break;
-    case QE_SRC_Q8_0: k_nl4_quant<QE_SRC_Q8_0><<<grid, block, 0, st>>>(a); break;
+    case QE_SRC_F32: go(k_nl4_quant<QE_SRC_F32, 3>, k_nl4_quant<QE_SRC_F32, 4>); break;
+    case QE_SRC_F16: go(k_nl4_quant<QE_SRC_F16, 3>, k_nl4_quant<QE_SRC_F16, 4>); break;
+    case QE_SRC_BF16: go(k_nl4_quant<QE_SRC_BF16, 3>, k_nl4_quant<QE_SRC_BF16, 4>); break;
+    case QE_SRC_Q8_0: go(k_nl4_quant<QE_SRC_Q8_0, 3>, k_nl4_quant<QE_SRC_Q8_0, 4>); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -1,0 +1,65 @@
+"""The converter's shortcut over the candidate scales, byte for byte against the oracle (needs an MI355X).
+
+Data on which the shortcut could go wrong: scales at both ends of the range it serves,
+integers and codebook values (elements exactly on midpoints), elements that change
+their entry exactly at a candidate, equal magnitudes, sparse and heavy-tailed blocks.
+The sizes are the smallest calls, a partly filled wave and both sides of the launch
+rule (768 workgroups of 256 blocks).
+"""
+import numpy as np
+import pytest
+
+import oracle as O
+import qe_moe
+
+pytestmark = pytest.mark.gpu
+KV = np.array([-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113], np.float64)
+MID = (KV[1:] + KV[:-1]) / 2
+
+
+def blocks(rng, n):
+    m = n // 10 + 1
+    z = lambda: rng.standard_normal((m, 32))  # noqa: E731
+    p = [z() * 10.0 ** rng.uniform(-8, 6, (m, 1)),                          # across both ends of [1e-6, 1e4]
+         z() * 10.0 ** rng.uniform(-6.3, -5.7, (m, 1)),
+         rng.integers(-127, 128, (m, 32)) * 2.0 ** rng.integers(-12, 3, (m, 1)),
+         rng.integers(-5, 6, (m, 32)) * rng.uniform(0.001, 1, (m, 1)),
+         rng.choice(np.concatenate([MID, KV]), (m, 32)) * rng.uniform(-0.1, 0.1, (m, 1)),
+         rng.standard_t(1.5, (m, 32)) * 0.02,
+         np.sign(z()) * rng.uniform(0.1, 2, (m, 1)),
+         z() * (rng.random((m, 32)) < 0.2)]
+    b = z()
+    b[:, 1:] *= rng.uniform(0.02, 0.12, (m, 1))                             # one large element
+    p.append(b)
+    top = rng.uniform(0.01, 1, (m, 1))
+    b = -rng.choice(MID, (m, 32)) * top / rng.integers(120, 135, (m, 32))   # on a midpoint at a candidate
+    b = np.where(np.abs(b) <= top, b, 0.0)
+    b[:, 0] = top[:, 0]
+    p.append(b)
+    x = np.concatenate(p).astype(np.float32)
+    return x[rng.permutation(len(x))[:n]]
+
+
+@pytest.mark.parametrize("src_type", [O.SRC_F32, O.SRC_BF16, O.SRC_Q8_0])
+@pytest.mark.parametrize("rows", [1, 37, 24576, 24577])
+def test_candidates_byte_exact(torch_cuda, src_type, rows):
+    torch = torch_cuda
+    print(f"converter candidates: type {src_type}, {rows} x 256", flush=True)
+    rng = np.random.default_rng(rows + src_type)
+    x = blocks(rng, rows * 8)
+    if src_type == O.SRC_F32:
+        src = x
+    elif src_type == O.SRC_BF16:
+        src = (x.view(np.uint32) >> 16).astype(np.uint16)
+    else:
+        d = np.abs(rng.standard_normal(len(x)) * 0.01).astype(np.float16)
+        q = rng.integers(-128, 128, (len(x), 32)).astype(np.int8)
+        q[::3] = rng.integers(-9, 10, q[::3].shape)
+        src = np.concatenate([d.view(np.uint8).reshape(-1, 2), q.view(np.uint8)], axis=1)
+    src = np.ascontiguousarray(src)
+    want = O.nl4_quantize_rows(src, src_type, rows, 256)
+    dev = torch.from_numpy(src.view(np.uint8).reshape(-1).copy()).cuda()
+    out = torch.full((rows * O.nl4_row_bytes(256),), 0xEE, dtype=torch.uint8, device="cuda")
+    qe_moe.nl4_quantize_rows(dev, src_type, rows, 256, out)
+    torch.cuda.synchronize()
+    assert np.array_equal(out.cpu().numpy().reshape(rows, -1), want)
