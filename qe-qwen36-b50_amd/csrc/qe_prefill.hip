@@ -1009,15 +1009,17 @@ template <int LEV> __global__ __launch_bounds__(256, 2) void k_router(const floa
 // block) and every wave reads its operands from there: each fetched byte feeds two
 // waves' MFMAs instead of one.  The Q8 block scales of the 128 rows sit in LDS for
 // the whole K, block-major, so the 32 rows a wave reads for one block are consecutive.
+// CH: blocks summed in one fma chain; a group of 2 CH blocks sums its halves apart.
 template <int S> struct Shgu64Smem {
     alignas(16) uint8_t a[S][2][2][4096]; // [group][stage][token tile][32-block of hi|lo halves, qe_hl_off order]
     alignas(16) uint8_t w[S][2][128][32]; // [group][stage][row: gate 0..63, up 64..127][32 int8]
     _Float16 sc[QE_D / 32][128];          // [block][row]
 };
-template <int S>
+template <int S, int CH>
 QE_DEV void shgu_tile64(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *hhl, int mp, int jg, Shgu64Smem<S> &sm) {
     constexpr uint32_t RB = QE_SH_GU_ROW_BYTES;
     constexpr int NB = QE_D / 32 / S; // blocks per group
+    static_assert(CH == NB || 2 * CH == NB, "one chain per group, or two");
     const int tid = threadIdx.x & 255, grp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), lane = tid & 63, wv = tid >> 6,
               c = lane & 31, kh = lane >> 5;
     const int mt32 = (T + 31) / 32, j0 = jg * 64, kb0 = grp * NB;
@@ -1065,7 +1067,7 @@ QE_DEV void shgu_tile64(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *
     fetch(1, st[1]);
     __syncthreads();
     const int ms = wv & 1, rg = 32 * (wv >> 1) + c, ru = 64 + rg;
-    qe_float16v ag = {}, au = {};
+    qe_float16v ag = {}, au = {}, ag0 = {}, au0 = {}; // ag0, au0: the first chain's sums
     // block b from stage s; block b + 2 is fetched, b + 1 put into the other stage
     auto block = [&](int b, int s) {
         fetch(b + 2 < NB ? b + 2 : NB - 1, st[s]);
@@ -1079,10 +1081,24 @@ QE_DEV void shgu_tile64(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *
         put(s ^ 1, st[s ^ 1]); // stage s ^ 1 was last read in block b - 1, before the barrier
         __syncthreads();
     };
+    static_assert(CH % 2 == 0, "a chain ends with a pair of stages");
 #pragma unroll 1
-    for (int b = 0; b < NB; b += 2) {
+    for (int b = 0; b < CH; b += 2) {
         block(b, 0);
         block(b + 1, 1);
+    }
+    if constexpr (CH < NB) {
+        ag0 = ag;
+        au0 = au;
+        ag = qe_float16v{};
+        au = qe_float16v{};
+#pragma unroll 1
+        for (int b = CH; b < NB; b += 2) {
+            block(b, 0);
+            block(b + 1, 1);
+        }
+        ag = ag0 + ag;
+        au = au0 + au;
     }
     static_assert(S == 1 || S == 2, "one group, or two whose sums meet");
     if constexpr (S == 2) { // the second group's sums through the activation stages
@@ -1117,12 +1133,13 @@ QE_DEV void shgu_tile64(const _Float16 *xhl, int T, const uint8_t *W, _Float16 *
     }
 }
 // workgroup b on XCD b % 8: the 8 row groups of one 64-token pair back to back there
-template <int S>
-__global__ __launch_bounds__(256 * S, 4) void k_shgu(const _Float16 *xhl, int T, const uint8_t *Wg, _Float16 *hhl) {
+// WPS: waves per SIMD the registers are cut for
+template <int S, int CH, int WPS>
+__global__ __launch_bounds__(256 * S, WPS) void k_shgu(const _Float16 *xhl, int T, const uint8_t *Wg, _Float16 *hhl) {
     __shared__ Shgu64Smem<S> sm;
     const int x = blockIdx.x & 7, k = blockIdx.x >> 3, mp = 8 * (k / 8) + x;
     if (mp >= (T + 63) / 64) return;
-    shgu_tile64<S>(xhl, T, Wg, hhl, mp, k % 8, sm);
+    shgu_tile64<S, CH>(xhl, T, Wg, hhl, mp, k % 8, sm);
 }
 
 // Shared down, 64 tokens x 128 output rows per workgroup: wave w takes token
@@ -1518,8 +1535,14 @@ hipError_t qe_launch_router_shgu(const QeLayerPtrs &L, const QeScratch &S, int T
         const int gs = 64 * (((T + 63) / 64 + 7) / 8);
         // below 4096 tokens the 64-token tiles alone leave CUs idle: two K groups per
         // tile (1999 tokens: 48 -> 35 us; at 8192 one group, four workgroups per CU)
-        if (T < 4096) k_shgu<2><<<gs, 512, 0, st>>>(S.xhl, T, L.sh_gu, (_Float16 *)S.shgu);
-        else k_shgu<1><<<gs, 256, 0, st>>>(S.xhl, T, L.sh_gu, (_Float16 *)S.shgu);
+        // Below 2048 a group sums in two chains of 16 blocks: one of 32 puts the shared
+        // expert's output 2.22e-7 from 64 bits (relative 2-norm), as against 1.98e-7.  There
+        // are at most 256 workgroups then, one per CU, so the second set of sums costs no
+        // occupancy (from 2048 on it would).
+        const auto shgu = [&](auto kern, int nt) { kern<<<gs, nt, 0, st>>>(S.xhl, T, L.sh_gu, (_Float16 *)S.shgu); };
+        if (T < 2048) shgu(k_shgu<2, 16, 2>, 512);
+        else if (T < 4096) shgu(k_shgu<2, 32, 4>, 512);
+        else shgu(k_shgu<1, 64, 4>, 256);
     } else { // XCD 0 has the most tiles of either kind
         const int grid = 8 * (rs_router_per_xcd(T, nz, 0) + rs_shgu_per_xcd(T, 0));
         const auto go = [&](auto kern) {
