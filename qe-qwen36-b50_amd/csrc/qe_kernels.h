@@ -25,16 +25,22 @@ static inline size_t qe_rpart_rows(size_t t_max) { // token rows of partials tha
 }
 #define QE_MFMA_MC 64 /* pairs per work item of the prefill MFMA grouped GEMMs (up to four 16-row tiles) */
 
-// Pairs per work item at T tokens.  Small calls fill the GPU with few workgroups, and
-// an expert's 33..64 pairs in one item made the longest of them (36 us alone, 50 in
-// company): items of 32 halve that (us per layer, skewed routing: 100 tokens 105 -> 88,
-// 200 tokens 113 -> 98).  With more tokens the second decode of the weights costs more
-// (250 tokens 106.6 -> 107.4, 400 tokens 155 -> 185).
+// Pairs per work item: QE_MFMA_MC, or 32 in a call of fewer than QE_ITEM32_T tokens
+// whose pairs fall on at most QE_ITEM32_E experts (k_disp_scatter counts them).  Few
+// experts leave the GPU partly empty, and then an expert's 33..64 pairs in one item make
+// the longest workgroups; items of 32 halve them.  With more experts the GPU is full and
+// the second decode of the weights costs more.  us per layer with items of 64 / 32:
+// 100 tokens over 66 experts 95 / 83; 200 tokens over 50 experts 100 / 89, over 98 97 / 93,
+// over 140 105 / 113; 223 tokens over 146 110 / 120.  In longer calls the line would have
+// to fall with T: 300 tokens over 105 experts 4 % slower, 400 over 80 11 %.
 #define QE_ITEM32_T 224
-static inline int qe_item_pairs(int T) { return T < QE_ITEM32_T ? 32 : QE_MFMA_MC; }
+#define QE_ITEM32_E 112
+static inline int qe_item32_experts(int T) { return T < QE_ITEM32_T ? QE_ITEM32_E : 0; }
 // upper bound of the items of T tokens: those of more than half the pairs, and one
 // smaller per expert
-static inline int qe_max_items(int T) { return T * QE_K_USED / (qe_item_pairs(T) / 2 + 1) + 1 + QE_N_EXPERT; }
+static inline int qe_max_items(int T) {
+    return T * QE_K_USED / ((qe_item32_experts(T) ? 32 : QE_MFMA_MC) / 2 + 1) + 1 + QE_N_EXPERT;
+}
 
 // One layer's weights inside the context.
 struct QeLayerPtrs {
