@@ -36,6 +36,17 @@ static inline size_t qe_rpart_rows(size_t t_max) { // token rows of partials tha
 #define QE_ITEM32_T 224
 #define QE_ITEM32_E 112
 static inline int qe_item32_experts(int T) { return T < QE_ITEM32_T ? QE_ITEM32_E : 0; }
+// Gate/up of items of up to 32 pairs: activations straight to registers (gu_small) where
+// more than qe_direct_experts(T) experts have pairs, staged through LDS elsewhere.  In
+// small calls, and over nearly all experts, items hold a few pairs each and their weights'
+// latency decides; with more pairs the four waves' separate reads of the activations cost
+// more than the staging.  us per layer direct / staged: 100 tokens over 248 experts 141 /
+// 147; 144 over 253 153 / 158, over 70 87 / 89; 180 over 132 106 / 95, over 94 96 / 89;
+// 223 over 103 107 / 98; 1000 over 256 260 / 241.
+#define QE_DIRECT_T 152  /* always direct below */
+#define QE_DIRECT_T2 256 /* never from here on */
+#define QE_DIRECT_E 224
+static inline int qe_direct_experts(int T) { return T < QE_DIRECT_T ? 0 : T < QE_DIRECT_T2 ? QE_DIRECT_E : QE_N_EXPERT; }
 // upper bound of the items of T tokens: those of more than half the pairs, and one
 // smaller per expert
 static inline int qe_max_items(int T) {
@@ -89,7 +100,7 @@ struct QeScratch {
     float *rpart;                           // [nz][T][256] router subtree partials (qe_router_splits)
     int32_t *ids; float *wts; float *shg;   // [T][8], [T][8], [T]
     int32_t *off; int32_t *pairs;           // [257], [T*8]
-    int4 *items; int32_t *n_items;          // work items (expert, first pair, count); n_items[0] items, the first n_items[1] of more than 32 pairs
+    int4 *items; int32_t *n_items;          // work items (expert, first pair, count); n_items[0] items, the first n_items[1] of more than 32 pairs; n_items[2]: small ones direct
     int8_t *hqp; float *hs;                 // [T*8][512] quantised h (operand layout), [T*8][16] scales
     float *sd;                              // [T][2048] shared-expert output
     float *yp;                              // [T*8][2048] weighted expert outputs

@@ -176,9 +176,10 @@ __global__ __launch_bounds__(1024) void k_disp_hist(const int32_t *ids, int np, 
 // in earlier waves plus its rank in its own wave (8 ballots on the id bits).
 // Block 0 also writes off[] and the work items (expert, first pair, count <= TC, 64, or
 // 32 where at most `few` experts have pairs): those of more than TC / 2 pairs first,
-// n_items[0] items in all, n_items[1] of them of more than 32 pairs.
+// n_items[0] items in all, n_items[1] of them of more than 32 pairs; n_items[2]: more than
+// `many` experts have pairs.
 __global__ __launch_bounds__(1024) void k_disp_scatter(const int32_t *ids, int np, const int32_t *chunk_hist, int nch,
-                                                       int few, int32_t *off_out, int32_t *pairs, int4 *items,
+                                                       int few, int many, int32_t *off_out, int32_t *pairs, int4 *items,
                                                        int32_t *n_items, int32_t *item_done) {
     __shared__ int s_before[QE_N_EXPERT], s_off[QE_N_EXPERT];
     __shared__ int s_w[16][QE_N_EXPERT];
@@ -209,13 +210,14 @@ __global__ __launch_bounds__(1024) void k_disp_scatter(const int32_t *ids, int n
     // items and large remainders), then the small remainders, each class in expert
     // order -- the longer items start first.
     __shared__ int s_wt[4][3], s_used[4];
-    int cnt = 0, full = 0, rem = 0, nb = 0, ns = 0, ic = 0, ib = 0, is = 0, tc = QE_MFMA_MC;
+    int cnt = 0, full = 0, rem = 0, nb = 0, ns = 0, ic = 0, ib = 0, is = 0, tc = QE_MFMA_MC, used = 0;
     if (tid < QE_N_EXPERT) cnt = (s_part[0][0][tid] + s_part[0][1][tid]) + (s_part[0][2][tid] + s_part[0][3][tid]);
-    if (few) {
-        const int used = __popcll(__ballot(cnt > 0));
-        if (tid < QE_N_EXPERT && lane == 0) s_used[wv] = used;
+    if (few || many < QE_N_EXPERT) {
+        const unsigned long long some = __ballot(cnt > 0);
+        if (tid < QE_N_EXPERT && lane == 0) s_used[wv] = __popcll(some);
         __syncthreads();
-        if ((s_used[0] + s_used[1]) + (s_used[2] + s_used[3]) <= few) tc = 32;
+        used = (s_used[0] + s_used[1]) + (s_used[2] + s_used[3]);
+        if (used <= few) tc = 32;
     }
     if (tid < QE_N_EXPERT) {
         s_before[tid] = (s_part[1][0][tid] + s_part[1][1][tid]) + (s_part[1][2][tid] + s_part[1][3][tid]);
@@ -268,6 +270,7 @@ __global__ __launch_bounds__(1024) void k_disp_scatter(const int32_t *ids, int n
         if (tid == QE_N_EXPERT - 1) {
             n_items[0] = all_b + all_s;
             n_items[1] = tc == QE_MFMA_MC ? all_b : 0; // of more than 32 pairs
+            n_items[2] = used > many;
         }
         if (item_done) // the fused gate/up + down launch counts its gate/up workgroups per item
             for (int i = tid; i < all_b + all_s; i += QE_N_EXPERT) item_done[i] = 0;
@@ -431,8 +434,8 @@ hipError_t qe_launch_layer(const QeLayerPtrs &L, const QeScratch &S, const float
     {
         QE_PROF(QP_DISPATCH); // the histogram came with k_topk
         const int np = T * QE_K_USED, nch = (np + 1023) / 1024;
-        k_disp_scatter<<<nch, 1024, 0, st>>>(S.ids, np, S.chunk_hist, nch, qe_item32_experts(T), S.off, S.pairs, S.items,
-                                              S.n_items, S.item_done);
+        k_disp_scatter<<<nch, 1024, 0, st>>>(S.ids, np, S.chunk_hist, nch, qe_item32_experts(T), qe_direct_experts(T), S.off,
+                                              S.pairs, S.items, S.n_items, S.item_done);
     }
     {
         QE_PROF(QP_GU); // routed gate/up, then routed down + shared down
@@ -452,7 +455,7 @@ hipError_t qe_launch_layer(const QeLayerPtrs &L, const QeScratch &S, const float
 hipError_t qe_launch_dispatch(const QeScratch &S, int T, hipStream_t st) {
     const int np = T * QE_K_USED, nch = (np + 1023) / 1024;
     k_disp_hist<<<nch, 1024, 0, st>>>(S.ids, np, S.chunk_hist);
-    k_disp_scatter<<<nch, 1024, 0, st>>>(S.ids, np, S.chunk_hist, nch, 0, S.off, S.pairs, S.items,
+    k_disp_scatter<<<nch, 1024, 0, st>>>(S.ids, np, S.chunk_hist, nch, 0, QE_N_EXPERT, S.off, S.pairs, S.items,
                                           S.n_items, nullptr);
     return hipGetLastError();
 }
@@ -509,7 +512,7 @@ hipError_t qe_launch_dispatch_noalloc(const int32_t *ids, int T, int32_t *off, i
     int32_t *n_items = (int32_t *)(base + NOALLOC_HIST_BYTES + (size_t)NOALLOC_ITEMS * 16);
     const int np = T * QE_K_USED, nch = (np + 1023) / 1024;
     k_disp_hist<<<nch, 1024, 0, st>>>(ids, np, chunk_hist);
-    k_disp_scatter<<<nch, 1024, 0, st>>>(ids, np, chunk_hist, nch, 0, off, pairs, items, n_items, nullptr);
+    k_disp_scatter<<<nch, 1024, 0, st>>>(ids, np, chunk_hist, nch, 0, QE_N_EXPERT, off, pairs, items, n_items, nullptr);
     return hipGetLastError();
 }
 

@@ -53,8 +53,8 @@ struct GemmTileArgs {
     const int8_t *aq;          // int8 activations in the operand layout (qe_opnd_off), row = token or pair
     int a_bytes;               // size of aq in bytes
     const float *as;           // their fp32 block scales
+    int direct;                // gate/up: small items take gu_small (1), or do where n_items[2] says so (2)
     int a_row_div;             // pair -> activation row: p / a_row_div (8 for tokens, 1 for pairs)
-    int direct;                // gate/up: small items take gu_small
     const int32_t *pairs;
     const int4 *items;         // (expert, first pair, count <= QE_MFMA_MC)
     const int32_t *n_items;
@@ -651,8 +651,8 @@ __device__ __forceinline__ void gu_small(const GemmTileArgs &a, const int4 it, c
 }
 
 // Gate/up: big items (33..64 pairs, the first n_items[1]) run NT = 4, NC = 2
-// on 8 row groups of 64 h rows; the small ones after them (NC = 1, or gu_small in
-// small calls) on 16 row groups of 32 h rows: twice the workgroups of half the life
+// on 8 row groups of 64 h rows; the small ones after them (NC = 1, or gu_small:
+// qe_direct_experts) on 16 row groups of 32 h rows: twice the workgroups of half the life
 // (these items run last, after the big ones, and their workgroups had made the
 // launch's tail).  Workgroup b runs on XCD x = b % 8 (round-robin dispatch) and
 // takes the (b / 8)-th row group of that XCD's items x, x + 8, ..., the big
@@ -672,7 +672,7 @@ QE_DEV void expert_unit(const GemmTileArgs &a, int b, ExpertSmem &sm) {
     static_assert(QE_MFMA_MC == 64, "items of up to four 16-row tiles");
     if (big)
         expert_tile<2, 4>(a, it, yb, sm);
-    else if (a.direct)
+    else if (a.direct == 1 || (a.direct == 2 && __builtin_amdgcn_readfirstlane(a.n_items[2])))
         it.z > 16 ? gu_small<2>(a, it, yb, sm) : gu_small<1>(a, it, yb, sm);
     else
         it.z > 16 ? expert_tile<1, 2>(a, it, yb, sm) : expert_tile<1, 1>(a, it, yb, sm);
@@ -1565,11 +1565,8 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
     GemmTileArgs g{};
     g.arena = L.arena; g.pairs = S.pairs; g.items = S.items; g.n_items = S.n_items; g.wts = S.wts;
     g.aq = S.xqp; g.a_bytes = T * QE_D; g.as = S.xs; g.a_row_div = QE_K_USED; g.hq = S.hqp; g.hs = S.hs;
-    // Below 256 tokens most items hold a few pairs and their weights' latency decides:
-    // activations straight to registers (100 tokens 157 -> 149 us).  With more pairs the
-    // four waves' separate reads of them cost more than the staging (1000 tokens 241 us
-    // staged, 260 direct).
-    g.direct = T < 256;
+    // a launch argument where T alone decides: the load costs 1 % of such a layer
+    g.direct = qe_direct_experts(T) == 0 ? 1 : qe_direct_experts(T) < QE_N_EXPERT ? 2 : 0;
     const bool fused = T >= QE_FUSE_T_MIN && T < QE_FUSE_T && S.item_done;
     if (fused) {
         g.item_done = S.item_done; g.err = S.err; g.err_val = S.err_val; g.spin_cap = S.spin_cap;

@@ -1,11 +1,11 @@
 """Prefill work items and gate/up forms at the sizes where the rule changes (needs an MI355X).
 
 Items hold up to 32 pairs in calls of fewer than 224 tokens over at most 112 experts and
-up to 64 in others; small items read their activations directly below 256 tokens and
-through LDS from there.  Eight hot experts take every token (items of 32 or 64 pairs and
-one remainder each), or the routing is flat (many items of a few pairs), or a given number
-of experts shares the pairs but for one that takes every token; the context is sized for
-exactly T tokens.
+up to 64 in others; small items read their activations directly below 152 tokens and,
+below 256, over more than 224 experts, and through LDS elsewhere.  Eight hot experts take
+every token (items of 32 or 64 pairs and one remainder each), or the routing is flat (many
+items of a few pairs), or a given number of experts shares the pairs but for one that takes
+every token; the context is sized for exactly T tokens.
 """
 import numpy as np
 import pytest
@@ -52,7 +52,8 @@ def test_items_at_rule_edges(torch_cuda, T, hot):
     check_layer(torch_cuda, T, bias)
 
 
-@pytest.mark.parametrize("T,used", [(96, 112), (96, 113), (128, 112), (129, 113), (223, 112), (223, 113), (224, 112)])
+@pytest.mark.parametrize("T,used", [(96, 112), (96, 113), (151, 112), (152, 112), (152, 113), (223, 112), (223, 113),
+                                    (224, 112), (223, 224), (223, 225), (255, 224), (255, 225), (256, 225)])
 def test_items_by_experts_used(torch_cuda, T, used):
     print(f"items at T={T} over {used} experts", flush=True)
     bias = np.zeros(256, np.float32)
