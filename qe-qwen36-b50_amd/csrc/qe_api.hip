@@ -139,8 +139,7 @@ int qe_moe_create(int device, int n_layers, int t_max, qe_moe_ctx **out) {
     c->have.assign(n_layers, 0u);
     c->have_exp.assign(n_layers, std::vector<uint8_t>(QE_N_EXPERT, 0));
     const size_t L = (size_t)n_layers, T = (size_t)t_max, NP = T * QE_K_USED, T32 = (T + 31) & ~(size_t)31;
-    size_t max_items = qe_max_items(t_max); // of any call of up to t_max tokens
-    if (t_max >= QE_ITEM32_T && max_items < (size_t)qe_max_items(QE_ITEM32_T - 1)) max_items = qe_max_items(QE_ITEM32_T - 1);
+    const size_t max_items = qe_max_items_upto(t_max);
     const size_t nch = (NP + 1023) / 1024;
     int rc = QE_OK;
     QeScratch &S = c->S;

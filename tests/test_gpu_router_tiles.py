@@ -49,6 +49,25 @@ def test_tiles_at_plan_edges(ctx, torch_cuda, T):
     assert np.linalg.norm(sd[pick] - ref_sd) <= 1e-5 * np.linalg.norm(ref_sd)
 
 
+@pytest.mark.parametrize("t_max,T", [(224, 223), (256, 255), (1280, 1279), (4096, 4095)])
+def test_call_that_needs_more_than_the_largest(torch_cuda, t_max, T):
+    """Contexts whose last call but one writes more items or router partials than the last
+    (the sizes themselves: test_plan_sizes.py)."""
+    print(f"t_max={t_max}, T={T}", flush=True)
+    L = O.SynthLayer(SEED, 0, bias=None)
+    m = qe_moe.MoE(n_layers=1, t_max=t_max)
+    try:
+        m.synth_layer(0, SEED, None)
+        for n in (T, t_max):
+            x = O.gen_x(SEED, 3000 + n, n)
+            lg, _ = run(torch_cuda, m, x)
+            ref = O.router(x, L.router, None)
+            assert np.array_equal(lg.view(np.uint32), ref.view(np.uint32))
+            m.check()
+    finally:
+        m.close()
+
+
 def q8_rows(raw, cols):
     raw = np.ascontiguousarray(raw).view(np.uint8).reshape(-1, cols + cols // 16)
     scale = np.ascontiguousarray(raw[:, cols:]).view(np.float16).astype(np.float64)
