@@ -40,6 +40,14 @@ def blocks(rng, n):
     return x[rng.permutation(len(x))[:n]]
 
 
+def convert(torch, src, src_type, rows):
+    dev = torch.from_numpy(np.ascontiguousarray(src).view(np.uint8).reshape(-1).copy()).cuda()
+    out = torch.full((rows * O.nl4_row_bytes(256),), 0xEE, dtype=torch.uint8, device="cuda")
+    qe_moe.nl4_quantize_rows(dev, src_type, rows, 256, out)
+    torch.cuda.synchronize()
+    return out.cpu().numpy().reshape(rows, -1)
+
+
 @pytest.mark.parametrize("src_type", [O.SRC_F32, O.SRC_BF16, O.SRC_Q8_0])
 @pytest.mark.parametrize("rows", [1, 37, 24576, 24577])
 def test_candidates_byte_exact(torch_cuda, src_type, rows):
@@ -56,10 +64,20 @@ def test_candidates_byte_exact(torch_cuda, src_type, rows):
         q = rng.integers(-128, 128, (len(x), 32)).astype(np.int8)
         q[::3] = rng.integers(-9, 10, q[::3].shape)
         src = np.concatenate([d.view(np.uint8).reshape(-1, 2), q.view(np.uint8)], axis=1)
-    src = np.ascontiguousarray(src)
-    want = O.nl4_quantize_rows(src, src_type, rows, 256)
-    dev = torch.from_numpy(src.view(np.uint8).reshape(-1).copy()).cuda()
-    out = torch.full((rows * O.nl4_row_bytes(256),), 0xEE, dtype=torch.uint8, device="cuda")
-    qe_moe.nl4_quantize_rows(dev, src_type, rows, 256, out)
-    torch.cuda.synchronize()
-    assert np.array_equal(out.cpu().numpy().reshape(rows, -1), want)
+    want = O.nl4_quantize_rows(np.ascontiguousarray(src), src_type, rows, 256)
+    assert np.array_equal(convert(torch, src, src_type, rows), want)
+
+
+# blocks out of the shortcut's range keep all fifteen candidates: in all lanes of a wave, in
+# about as many as decide between the two ways of evaluating them (48 of 64), or in half;
+# 37 rows end in a wave of 40 blocks
+@pytest.mark.parametrize("rows", [37, 24577])
+@pytest.mark.parametrize("scale,share", [(3e-8, 1.0), (2e-7, 1.0), (1e5, 1.0), (1e-7, 0.75), (1e5, 0.74), (1e-7, 0.5)])
+def test_blocks_out_of_range(torch_cuda, scale, share, rows):
+    print(f"converter out of range: {scale}, {share} of the blocks, {rows} x 256", flush=True)
+    rng = np.random.default_rng(rows)
+    n = rows * 8
+    x = rng.standard_normal((n, 32)) * np.where(rng.random((n, 1)) < share, scale, 0.02)
+    x = x.astype(np.float32)
+    want = O.nl4_quantize_rows(x, O.SRC_F32, rows, 256)
+    assert np.array_equal(convert(torch_cuda, x, O.SRC_F32, rows), want)
