@@ -2,7 +2,8 @@
 
 Data on which the shortcut could go wrong: scales at both ends of the range it serves,
 integers and codebook values (elements exactly on midpoints), elements that change
-their entry exactly at a candidate, equal magnitudes, sparse and heavy-tailed blocks.
+their entry exactly at a candidate, equal magnitudes, sparse and heavy-tailed blocks,
+blocks outside the range, NaN and infinities.
 The sizes are the smallest calls, a partly filled wave and both sides of the launch
 rule (768 workgroups of 256 blocks).
 """
@@ -48,7 +49,7 @@ def convert(torch, src, src_type, rows):
     return out.cpu().numpy().reshape(rows, -1)
 
 
-@pytest.mark.parametrize("src_type", [O.SRC_F32, O.SRC_BF16, O.SRC_Q8_0])
+@pytest.mark.parametrize("src_type", [O.SRC_F32, O.SRC_F16, O.SRC_BF16, O.SRC_Q8_0])
 @pytest.mark.parametrize("rows", [1, 37, 24576, 24577])
 def test_candidates_byte_exact(torch_cuda, src_type, rows):
     torch = torch_cuda
@@ -57,6 +58,8 @@ def test_candidates_byte_exact(torch_cuda, src_type, rows):
     x = blocks(rng, rows * 8)
     if src_type == O.SRC_F32:
         src = x
+    elif src_type == O.SRC_F16:
+        src = np.clip(x, -60000, 60000).astype(np.float16)
     elif src_type == O.SRC_BF16:
         src = (x.view(np.uint32) >> 16).astype(np.uint16)
     else:
@@ -81,3 +84,25 @@ def test_blocks_out_of_range(torch_cuda, scale, share, rows):
     x = x.astype(np.float32)
     want = O.nl4_quantize_rows(x, O.SRC_F32, rows, 256)
     assert np.array_equal(convert(torch_cuda, x, O.SRC_F32, rows), want)
+
+
+@pytest.mark.parametrize("rows", [37, 24577])
+def test_nan_and_infinities(torch_cuda, rows):
+    """A block with a NaN or an infinity has a NaN scale (its codes are not defined), and
+    leaves its neighbours in the wave as they are."""
+    print(f"converter NaN and infinities: {rows} x 256", flush=True)
+    rng = np.random.default_rng(rows)
+    n = rows * 8
+    x = (rng.standard_normal((n, 32)) * 0.02).astype(np.float32)
+    for step, first, value in ((5, 0, np.nan), (7, 1, np.inf), (11, 2, -np.inf)):
+        at = np.arange(first, n, step)
+        x[at, rng.integers(0, 32, at.size)] = value
+    bad = ~np.isfinite(x).all(axis=1)
+    with np.errstate(all="ignore"):
+        want = O.nl4_quantize_rows(x, O.SRC_F32, rows, 256)
+    got = convert(torch_cuda, x, O.SRC_F32, rows)
+    codes = [r[:, :128].reshape(n, 16) for r in (got, want)]
+    scales = [np.ascontiguousarray(r[:, 128:]).view(np.float16).reshape(n) for r in (got, want)]
+    assert np.array_equal(codes[0][~bad], codes[1][~bad])
+    assert np.array_equal(scales[0][~bad].view(np.uint16), scales[1][~bad].view(np.uint16))
+    assert np.isnan(scales[1][bad]).all() and np.isnan(scales[0][bad]).all()
