@@ -27,15 +27,17 @@
 //     reaches).  Each change is added to the bin of its n; prefix sums over the bins give
 //     S_xq and S_qq of every candidate.  All their terms have one sign (bar an opposite
 //     entry 1, below 1e-4 of the sum), so the relative errors are at most the roundings
-//     on a term's way, of 2^-24 each: 2 + 31 in the sequence, 2 + 8 + 2 + 14 here, and up
-//     to 31 more on what met in one bin (at most 0.21 of S_xq and 0.35 of S_qq).
+//     on a term's way, of 2^-24 each: 3 + 31 in the sequence, 2 + 8 + 2 + 14 here, and up
+//     to 31 more on what met in one bin (at most 0.21 of S_xq and 0.36 of S_qq).
 //   * A candidate whose approximate score S_xq^2 / S_qq is below the largest by more than
-//     3e-5 (2 x 99 roundings of the sequence's score, 2 x 102 of this one: 2.4e-5, and the
+//     3e-5 (2 x 102 roundings of the sequence's score, 2 x 102 of this one: 2.4e-5, and the
 //     last operations) cannot be the last to win; what is left -- mostly one candidate --
 //     is evaluated with the fp32 operations of the sequence, in its order, starting from
 //     s0's exact score.  The first is evaluated by the block's own lane, the others by the
 //     wave's lanes in turn.  Candidates with no change between them assign alike and
-//     score alike, and only the first is evaluated.
+//     score alike, and only the first is evaluated.  (No change is lost in S_xq's sum: the
+//     smallest adds 11 (4.5/134)^3 |m|^3 = 4.2e-4 |m|^3, and half an ulp of the largest sum,
+//     32 x 127 |m|^3, is at most 2.5e-4 |m|^3.  A test of the bin alone spills registers.)
 //   * Blocks whose largest element lies outside [1e-6, 1e4], where the products could
 //     underflow or overflow, or that hold a NaN, take the sequence over all sixteen.
 //

@@ -86,6 +86,25 @@ def test_blocks_out_of_range(torch_cuda, scale, share, rows):
     assert np.array_equal(convert(torch_cuda, x, O.SRC_F32, rows), want)
 
 
+def test_smallest_change_beside_the_largest_sum(torch_cuda):
+    """31 elements (or 24 to 30) of the largest magnitude, and a few that change their entry
+    at the smallest midpoint, -4.5, at one of the candidates or an ulp or two beside it: the
+    change is 1e-7 of the sum, and which side of it wins is a matter of roundings."""
+    rows = 513
+    print(f"converter smallest change, {rows} x 256", flush=True)
+    rng = np.random.default_rng(5)
+    n = rows * 8
+    m = (rng.uniform(0.5, 1, (n, 1)) * 10.0 ** rng.uniform(-5, 3, (n, 1))).astype(np.float32)
+    x = np.repeat(m, 32, axis=1)
+    k = rng.choice([1, 1, 2, 4, 8], n)
+    small = (4.5 * m.astype(np.float64) / rng.integers(119, 136, (n, 32))).astype(np.float32)
+    small = (small.view(np.int32) + rng.integers(-2, 3, (n, 32), dtype=np.int32)).view(np.float32)
+    x = np.where(np.arange(32)[None, :] >= 32 - k[:, None], small, x)
+    x *= rng.choice([-1, 1], (n, 1)).astype(np.float32)
+    want = O.nl4_quantize_rows(x, O.SRC_F32, rows, 256)
+    assert np.array_equal(convert(torch_cuda, x, O.SRC_F32, rows), want)
+
+
 @pytest.mark.parametrize("rows", [37, 24577])
 def test_nan_and_infinities(torch_cuda, rows):
     """A block with a NaN or an infinity has a NaN scale (its codes are not defined), and
