@@ -177,7 +177,7 @@ __global__ __launch_bounds__(1024) void k_disp_hist(const int32_t *ids, int np, 
 // Block 0 also writes off[] and the work items (expert, first pair, count <= TC, 64, or
 // 32 where at most `few` experts have pairs): those of more than TC / 2 pairs first,
 // n_items[0] items in all, n_items[1] of them of more than 32 pairs; n_items[2]: more than
-// `many` experts have pairs.
+// `many` experts have pairs (for many 1..255).
 __global__ __launch_bounds__(1024) void k_disp_scatter(const int32_t *ids, int np, const int32_t *chunk_hist, int nch,
                                                        int few, int many, int32_t *off_out, int32_t *pairs, int4 *items,
                                                        int32_t *n_items, int32_t *item_done) {
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(1024) void k_disp_scatter(const int32_t *ids, int n
     __shared__ int s_wt[4][3], s_used[4];
     int cnt = 0, full = 0, rem = 0, nb = 0, ns = 0, ic = 0, ib = 0, is = 0, tc = QE_MFMA_MC, used = 0;
     if (tid < QE_N_EXPERT) cnt = (s_part[0][0][tid] + s_part[0][1][tid]) + (s_part[0][2][tid] + s_part[0][3][tid]);
-    if (few || many < QE_N_EXPERT) {
+    if (few || (many > 0 && many < QE_N_EXPERT)) {
         const unsigned long long some = __ballot(cnt > 0);
         if (tid < QE_N_EXPERT && lane == 0) s_used[wv] = __popcll(some);
         __syncthreads();

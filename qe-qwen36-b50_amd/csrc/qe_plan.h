@@ -37,9 +37,10 @@ static inline size_t qe_rpart_rows(size_t t_max) {
 // 100 tokens over 66 experts 95 / 83; 200 tokens over 50 experts 100 / 89, over 98 97 / 93,
 // over 140 105 / 113; 223 tokens over 146 110 / 120.  In longer calls the line would have
 // to fall with T: 300 tokens over about 110 experts 10 % slower, 400 over about 85 11 %.
+// (Up to 16 tokens no expert has more than 16 pairs and the items are the same either way.)
 #define QE_ITEM32_T 224
 #define QE_ITEM32_E 112
-static inline int qe_item32_experts(int T) { return T < QE_ITEM32_T ? QE_ITEM32_E : 0; }
+static inline int qe_item32_experts(int T) { return T > 16 && T < QE_ITEM32_T ? QE_ITEM32_E : 0; }
 
 // Gate/up of items of up to 32 pairs: activations straight to registers (gu_small) where
 // more than qe_direct_experts(T) experts have pairs, staged through LDS elsewhere.  In

@@ -669,9 +669,11 @@ QE_DEV void expert_unit(const GemmTileArgs &a, int b, ExpertSmem &sm) {
     if (item >= a.n_items[0]) return;
     const int4 it = a.items[item];
     static_assert(QE_MFMA_MC == 64, "items of up to four 16-row tiles");
+    int direct = a.direct;
+    if (direct == 2) direct = __builtin_amdgcn_readfirstlane(a.n_items[2]);
     if (big)
         expert_tile<2, 4>(a, it, yb, sm);
-    else if (a.direct == 1 || (a.direct == 2 && __builtin_amdgcn_readfirstlane(a.n_items[2])))
+    else if (direct)
         it.z > 16 ? gu_small<2>(a, it, yb, sm) : gu_small<1>(a, it, yb, sm);
     else
         it.z > 16 ? expert_tile<1, 2>(a, it, yb, sm) : expert_tile<1, 1>(a, it, yb, sm);

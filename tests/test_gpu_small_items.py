@@ -42,7 +42,7 @@ def check_layer(torch, T, bias, used=None):
 
 
 @pytest.mark.parametrize("hot", [True, False])
-@pytest.mark.parametrize("T", [9, 31, 32, 97, 223, 224, 255, 256])
+@pytest.mark.parametrize("T", [9, 16, 17, 31, 32, 97, 151, 152, 223, 224, 255, 256])
 def test_items_at_rule_edges(torch_cuda, T, hot):
     print(f"items at T={T}, {'8 hot experts' if hot else 'flat routing'}", flush=True)
     bias = None
