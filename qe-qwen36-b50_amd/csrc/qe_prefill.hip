@@ -54,6 +54,7 @@ struct GemmTileArgs {
     int a_bytes;               // size of aq in bytes
     const float *as;           // their fp32 block scales
     int direct;                // gate/up: small items take gu_small (1), or do where n_items[2] says so (2)
+    int a_row_div;             // pair -> activation row: p / a_row_div (8 for tokens, 1 for pairs)
     const int32_t *pairs;
     const int4 *items;         // (expert, first pair, count <= QE_MFMA_MC)
     const int32_t *n_items;
@@ -289,14 +290,14 @@ __device__ __forceinline__ void expert_tile(const GemmTileArgs &a, const int4 it
 #pragma unroll
     for (int r = 0; r < NPASS; ++r) {
         const int m = 32 * r + (tid >> 3), p = m < 16 * NT ? s_pair[m] : -1;
-        act_off[r] = (uint32_t)((p < 0 ? s_pair[0] : p) / QE_K_USED) * KD + 16 * (tid & 7);
+        act_off[r] = (uint32_t)((p < 0 ? s_pair[0] : p) / a.a_row_div) * KD + 16 * (tid & 7);
     }
     const bool act_role = 32 * (NPASS - 1) + (tid >> 3) < 16 * NT; // the last pass (all passes when NT > 1)
     const int act_st = (tid >> 3) * 128 + (((tid & 7) ^ ((tid >> 4) & 7)) << 4); // + 32 r * 128
     const int xs_m = tid - (256 - 16 * NT);
     const bool xs_role = xs_m >= 0;
     const int xs_p = xs_role ? s_pair[xs_m] : -1;
-    const float4 *xs_src = (const float4 *)(a.as + (size_t)((xs_p < 0 ? 0 : xs_p) / QE_K_USED) * NB);
+    const float4 *xs_src = (const float4 *)(a.as + (size_t)((xs_p < 0 ? 0 : xs_p) / a.a_row_div) * NB);
     uint4 sa[NPASS];
     float4 sxs = make_float4(0.f, 0.f, 0.f, 0.f);
     auto stage_load = [&](int qq) {
@@ -1565,7 +1566,7 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
     const int np = T * QE_K_USED;
     GemmTileArgs g{};
     g.arena = L.arena; g.pairs = S.pairs; g.items = S.items; g.n_items = S.n_items; g.wts = S.wts;
-    g.aq = S.xqp; g.a_bytes = T * QE_D; g.as = S.xs; g.hq = S.hqp; g.hs = S.hs;
+    g.aq = S.xqp; g.a_bytes = T * QE_D; g.as = S.xs; g.a_row_div = QE_K_USED; g.hq = S.hqp; g.hs = S.hs;
     // a launch argument where T alone decides: the load costs 1 % of such a layer
     g.direct = qe_direct_experts(T) == 0 ? 1 : qe_direct_experts(T) < QE_N_EXPERT ? 2 : 0;
     const bool fused = T >= QE_FUSE_T_MIN && T < QE_FUSE_T && S.item_done;
@@ -1576,7 +1577,7 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
         k_expert_gu<<<expert_max_wg(T), 256, 0, st>>>(g);
     }
     GemmTileArgs d = g;
-    d.aq = S.hqp; d.a_bytes = np * QE_FF_EXP; d.as = S.hs; d.yp = S.yp;
+    d.aq = S.hqp; d.a_bytes = np * QE_FF_EXP; d.as = S.hs; d.a_row_div = 1; d.yp = S.yp;
     // row groups per down workgroup: fewer, longer workgroups where the items
     // alone fill the CUs several times over
     // (4 from 256 tokens in separate launches: measured best at 512 and 8192; fused,
