@@ -54,7 +54,9 @@ struct GemmTileArgs {
     int a_bytes;               // size of aq in bytes
     const float *as;           // their fp32 block scales
     int direct;                // gate/up: small items take gu_small (1), or do where n_items[2] says so (2)
-    int a_row_div;             // pair -> activation row: p / a_row_div (8 for tokens, 1 for pairs)
+    // pairs per token, 8, read by gate/up.  As the constant it is, the staged tiles'
+    // start-up compiles to slower code (layer of 512 tokens 135.0 -> 136.0 us).
+    int a_row_div;
     const int32_t *pairs;
     const int4 *items;         // (expert, first pair, count <= QE_MFMA_MC)
     const int32_t *n_items;
@@ -1577,7 +1579,7 @@ hipError_t qe_launch_expert_mfma(const QeLayerPtrs &L, const QeScratch &S, int T
         k_expert_gu<<<expert_max_wg(T), 256, 0, st>>>(g);
     }
     GemmTileArgs d = g;
-    d.aq = S.hqp; d.a_bytes = np * QE_FF_EXP; d.as = S.hs; d.a_row_div = 1; d.yp = S.yp;
+    d.aq = S.hqp; d.a_bytes = np * QE_FF_EXP; d.as = S.hs; d.yp = S.yp;
     // row groups per down workgroup: fewer, longer workgroups where the items
     // alone fill the CUs several times over
     // (4 from 256 tokens in separate launches: measured best at 512 and 8192; fused,
