@@ -33,13 +33,14 @@
 //     3e-5 (2 x 102 roundings of the sequence's score, 2 x 102 of this one: 2.4e-5, and the
 //     last operations) cannot be the last to win; what is left -- mostly one candidate --
 //     is evaluated with the fp32 operations of the sequence, in its order, starting from
-//     s0's exact score.  The first is evaluated by the block's own lane, the others by the
-//     wave's lanes in turn.  Candidates with no change between them assign alike and
+//     s0's exact score.  The first is evaluated by the block's own lane, the others -- about
+//     one block in three has any -- by the wave's lanes in turn.  Candidates with no change between them assign alike and
 //     score alike, and only the first is evaluated.  (No change is lost in S_xq's sum: the
 //     smallest adds 11 (4.5/134)^3 |m|^3 = 4.2e-4 |m|^3, and half an ulp of the largest sum,
 //     32 x 127 |m|^3, is at most 2.5e-4 |m|^3.  A test of the bin alone spills registers.)
 //   * Blocks whose largest element lies outside [1e-6, 1e4], where the products could
-//     underflow or overflow, or that hold a NaN, take the sequence over all sixteen.
+//     underflow or overflow, or that hold a NaN, take the sequence over all sixteen.  Where
+//     three lanes of a wave in four have such a block, each evaluates its own.
 //
 // nearest(a): ggml bisects the codebook and keeps the lower of the two
 // bracketing entries when a - lo < hi - a.  Both differences are exact
@@ -155,13 +156,14 @@ __device__ inline float scale8(float n, float mn, float rn) {
     return fmaf(fmaf(-q, mn, n), rn, q);
 }
 
-// WPS: waves per SIMD the registers are cut for (qe_launch_nl4_quant).
-// What bounds it: VALU issue (3,075 instructions a block of 64 threads, of half rate
-// where they convert, clamp or mask) and the slot reads' bank conflicts (a third of the
-// cycles).  One Q8_0 layer (25 M blocks): 2,440 us scoring all candidates, 1,590 now;
-// 16,384 bf16 blocks 14.8 -> 11.5 us.  Measured on the way: the bins by LDS float atomics
-// 9,020 us; every lane evaluating its own remaining candidates 1,750 (four rounds a wave
-// instead of about 1.4).
+// WPS: waves per SIMD the registers are cut for (qe_launch_nl4_quant).  At four, F16
+// spills 6 VGPRs and BF16 one (16 and 8 bytes of scratch a lane); F32 and Q8_0 none.
+// What bounds it: VALU issue (3,090 instructions a wave of 64 blocks, of half rate where
+// they convert, clamp or mask) and the slot reads' bank conflicts (36 % of the cycles).
+// One Q8_0 layer (25 M blocks): 2,455 us scoring all candidates, 1,590 now; 32,768 bf16
+// blocks 14.8 -> 11.7 us.  Measured on the way: the bins by LDS float atomics 9,020 us;
+// every lane evaluating its own remaining candidates 1,750 (four rounds a wave instead of
+// about 1.4).
 template <int TYPE, int WPS>
 __global__ __launch_bounds__(256, WPS) void k_nl4_quant(QeNl4Args a) {
     constexpr int N0 = 120, NC = 15; // candidates s = -n/m, n = N0 .. N0 + NC - 1 (t = 127 - n)
@@ -333,7 +335,7 @@ hipError_t qe_launch_nl4_quant(const QeNl4Args &a, int src_type, hipStream_t st)
     if (a.nblk == 0) return hipSuccess;
     const dim3 grid((a.nblk + 255) / 256), block(256);
     // up to three workgroups per CU: all run at once, and what counts is one wave's own
-    // pace, which more registers help (16,384 blocks 13.0 -> 11.5 us); beyond, the fourth
+    // pace, which more registers help (32,768 blocks 13.0 -> 11.5 us); beyond, the fourth
     // wave per SIMD does (25 M blocks 1,727 -> 1,590)
     const auto go = [&](auto small, auto large) {
         if (grid.x <= 3 * 256) small<<<grid, block, 0, st>>>(a);

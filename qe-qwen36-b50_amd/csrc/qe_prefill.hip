@@ -1494,6 +1494,11 @@ __global__ __launch_bounds__(256, 2) void k_expert_dn(GemmTileArgs a, int nr, in
 // through, sc1, and acknowledged first) and stages h from the coherence point.
 // The dispatcher starts an XCD's workgroups in grid order, so every gate/up
 // workgroup a down one waits for has started.
+// Layer us one launch / two: flat routing 16 tokens 69 / 74, 32 tokens 97 / 101, 100 tokens
+// 142 / 145; 64 tokens over 93 experts 76 / 79.  The lower line was drawn on slower down
+// tiles, and it is a line in T where the experts with pairs decide: over fewer of them two
+// launches are the faster at every size up to 256 (32 tokens over 45 experts 79 / 61, 100
+// over 36 92 / 74, 256 over 47 100 / 90; 12 tokens over 40 70 / 54).
 #ifndef QE_FUSE_T_MIN
 #define QE_FUSE_T_MIN 32
 #endif
